@@ -42,7 +42,10 @@
 // Causal work is uneven across query tiles: the grid runs the last (most
 // keys) tiles of every head first.
 //
-// attn_prefill_generic<T>: f32 storage, and half storage with other D: one
+// attn_prefill_f32<D>: f32 storage, D in {64, 128}, 16-byte aligned: the same
+// products on the float32 matrix instructions (described there).
+//
+// attn_prefill_generic<T>: every other D and alignment: one
 // wave per query row, lanes across D in float4 chunks, online softmax over
 // the keys (a parity path).
 #include "ft_common.hpp"
@@ -54,6 +57,8 @@ namespace ft {
 namespace {
 
 constexpr float kLog2eP = 1.4426950408889634f;
+constexpr float kLog2eLo = 1.925963033500e-8f;  // log2(e) - kLog2eP
+constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kPQ = 128;                  // query rows per workgroup
 constexpr int kPKV = 64;                  // key rows per tile
 constexpr float kLazy = 8.0f;             // log2 of the largest unnormalised weight
@@ -509,30 +514,19 @@ void attn_prefill_mfma(const T* __restrict__ q, const T* __restrict__ k,
     }
 }
 
-// one wave per (b, q head, query row); lanes hold float4 chunks c = lane,
-// lane + 64 of D
+// one query row by one wave: qr its query, kh / vh its kv head's rows, lim the
+// keys it attends; lanes hold float4 chunks c = lane, lane + 64 of D
 template <typename T>
-__global__ __launch_bounds__(64) void attn_prefill_generic(
-    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
-    T* __restrict__ out, int hq, int hkv, int seq, int dim, int causal, float scale) {
-    const long long id = blockIdx.x;
-    const int i = (int)(id % seq);
-    const long long bh = id / seq;
-    const int h = (int)(bh % hq);
-    const long long b = bh / hq;
-    const int kvh = h / (hq / hkv);
-    const int lane = threadIdx.x;
+__device__ __forceinline__ void prefill_row(const T* __restrict__ qr, const T* __restrict__ kh,
+                                            const T* __restrict__ vh, T* __restrict__ orow,
+                                            int lim, int dim, float scale, int lane) {
     const int nc = dim / 4;
-    const T* qr = q + ((size_t)bh * seq + i) * dim;
-    const T* kh = k + ((size_t)b * hkv + kvh) * seq * dim;
-    const T* vh = v + ((size_t)b * hkv + kvh) * seq * dim;
     const bool c0 = lane < nc, c1 = lane + 64 < nc;
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
     const float4 q0 = c0 ? St<T>::ld4(qr + 4 * lane) : z;
     const float4 q1 = c1 ? St<T>::ld4(qr + 4 * (lane + 64)) : z;
     float4 a0 = z, a1 = z;
     float m = -INFINITY, l = 0.f;
-    const int lim = causal ? i + 1 : seq;
     for (int t = 0; t < lim; ++t) {
         const T* kr = kh + (size_t)t * dim;
         float d = 0.f;
@@ -563,11 +557,281 @@ __global__ __launch_bounds__(64) void attn_prefill_generic(
         }
     }
     const float inv = 1.0f / l;
-    T* orow = out + ((size_t)bh * seq + i) * dim;
     if (c0) St<T>::st4(orow + 4 * lane, make_float4(a0.x * inv, a0.y * inv, a0.z * inv, a0.w * inv));
     if (c1)
         St<T>::st4(orow + 4 * (lane + 64),
                    make_float4(a1.x * inv, a1.y * inv, a1.z * inv, a1.w * inv));
+}
+
+// one wave per (b, q head, query row)
+template <typename T>
+__global__ __launch_bounds__(64) void attn_prefill_generic(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
+    T* __restrict__ out, int hq, int hkv, int seq, int dim, int causal, float scale) {
+    const long long id = blockIdx.x;
+    const int i = (int)(id % seq);
+    const long long bh = id / seq;
+    const int h = (int)(bh % hq);
+    const long long b = bh / hq;
+    const int kvh = h / (hq / hkv);
+    const size_t kv0 = ((size_t)b * hkv + kvh) * seq * dim;
+    const size_t row = ((size_t)bh * seq + i) * dim;
+    prefill_row<T>(q + row, k + kv0, v + kv0, out + row, causal ? i + 1 : seq, dim, scale,
+                   threadIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// float32, D in {64, 128}: the same transposed products on
+// v_mfma_f32_16x16x4_f32 (lane (r, g): A[r][g], B[g][r], C[4g+i][r]), so
+// every product and sum is float32 as in prefill_row.
+//
+// What bounds it: the float32 matrix rate (256 flop / clock / CU, 1/16 of
+// bf16). A workgroup owns 64 query rows (16 a wave) of one (b, q head) and
+// walks 64-key tiles: at D = 128 a tile is 8192 MFMA cycles a wave against
+// 512 LDS cycles for its K and V reads, so operand reuse is not the point and
+// the query tile is kept small for balance (with 128 rows the longest
+// causal workgroup of a 1500-token prompt alone takes 164 us).
+// The next tile waits in registers while this one is multiplied; two
+// workgroups a CU (67 KB of LDS each at D = 128) cover each other's softmax
+// and barriers.
+//
+//   scores  S^T[key][q]: lane (r, g) reads K[key r][16j + 4g .. +3] with one
+//           ds_read_b128 (rows padded by 16 bytes: conflict-free) and feeds
+//           4 MFMAs, whose k slot g is dim 16j + 4g + c; Q likewise, in
+//           registers. Lane (q, g) gets keys 4g + i of a 16-key block.
+//   PV      O^T[d][q]: MFMA i of a key block takes the weight the lane
+//           already holds for key 4g + i as B; A is V[key 4g + i][64h + 4r
+//           .. +3] (one ds_read_b128, a whole 256-byte half row per 16
+//           lanes), output row r of MFMA (h, c) being dim 64h + 4r + c. The
+//           lane ends up with dims 64h + 16g + 4i + c: float4 stores.
+//
+// A masked key's weight is 0, and 0 * inf is not: where a tile that crosses
+// the diagonal holds a V value that is not finite, the workgroup's rows are
+// computed again by prefill_row, which touches the attended keys alone.
+//
+// Measured (32 / 8 heads, D = 128, S = 1500, causal): 4013 us a call with
+// one wave per query row (attn_prefill_generic), 205 us here (MFMA busy 57% of
+// the cycles, 65% of those a CU has a workgroup). 32-key tiles with three
+// workgroups a CU: 240 us (all 768 workgroups start at once, the long ones
+// share their CUs to the end). Error against 64 bits 3.1e-7, 3.8e-7 before.
+// ---------------------------------------------------------------------------
+constexpr int kFT = 64;  // query rows per workgroup, keys per tile
+
+template <int D>
+__global__ __launch_bounds__(256, 2)
+void attn_prefill_f32(const float* __restrict__ q, const float* __restrict__ k,
+                      const float* __restrict__ v, float* __restrict__ out, int batch, int hq,
+                      int hkv, int seq, int causal, float scale) {
+    constexpr int kPitch = D + 4;              // floats per K row in LDS
+    constexpr int kCh = D / 4;                 // 16-byte chunks per row
+    constexpr int kLoads = kFT * kCh / 256;    // chunks per thread and tile
+    constexpr int kJ = D / 16, kH = D / 64;
+    __shared__ __attribute__((aligned(16))) float ks[kFT * kPitch];
+    __shared__ __attribute__((aligned(16))) float vs[kFT * D];
+
+    // blocks go round the 8 XCDs: each XCD takes a run of consecutive heads,
+    // so the q heads of one kv head read K and V through one L2
+    const int nqt = (seq + kFT - 1) / kFT;
+    const unsigned nbh = (unsigned)(batch * hq);
+    const int qt = nqt - 1 - (int)(blockIdx.x / nbh);
+    unsigned bh = blockIdx.x % nbh;
+    if (nbh % 8 == 0) bh = (bh & 7) * (nbh >> 3) + (bh >> 3);
+    const int b = (int)(bh / hq), h = (int)(bh - (unsigned)b * hq);
+    const int kvh = h / (hq / hkv);
+    const int q0 = qt * kFT;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int wrow0 = q0 + 16 * wave;
+
+    const float* qh = q + (size_t)bh * seq * D;
+    const float* kh = k + ((size_t)b * hkv + kvh) * seq * D;
+    const float* vh = v + ((size_t)b * hkv + kvh) * seq * D;
+
+    f32x4 qf[kJ];
+    {
+        const float* qr = qh + (size_t)min(wrow0 + r, seq - 1) * D + 4 * g;
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) qf[j] = *reinterpret_cast<const f32x4*>(qr + 16 * j);
+    }
+
+    const int nkv = (seq + kFT - 1) / kFT;
+    const int nkt = causal ? min(nkv, qt + 1) : nkv;
+
+    f32x4 kreg[kLoads], vreg[kLoads];
+    auto load_tile = [&](int kt) {  // rows past the sequence are zeros
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int c = tid + 256 * j;
+            const int row = kt * kFT + c / kCh;
+            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            const size_t off = (size_t)min(row, seq - 1) * D + 4 * (c % kCh);
+            const f32x4 kk = *reinterpret_cast<const f32x4*>(kh + off);
+            const f32x4 vv = *reinterpret_cast<const f32x4*>(vh + off);
+            kreg[j] = row < seq ? kk : z;
+            vreg[j] = row < seq ? vv : z;
+        }
+    };
+    auto store_tile = [&]() {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int c = tid + 256 * j;
+            *reinterpret_cast<f32x4*>(ks + (c / kCh) * kPitch + 4 * (c % kCh)) = kreg[j];
+            *reinterpret_cast<f32x4*>(vs + 4 * c) = vreg[j];
+        }
+    };
+
+    f32x4 o[kH][4];
+#pragma unroll
+    for (int hh = 0; hh < kH; ++hh)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[hh][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;
+    // scale * log2(e) in two parts
+    const float scale_log2 = scale * kLog2eP;
+    const float lo_ln2 = kLn2 * (fmaf(scale, kLog2eP, -scale_log2) + scale * kLog2eLo);
+    const float lazy_raw = kLazy / scale_log2;
+    int bad = 0;  // a masked V value that is not finite
+
+    load_tile(0);
+    for (int kt = 0; kt < nkt; ++kt) {
+        const int kv0 = kt * kFT;
+        if (causal && kt == qt) {
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    bad |= (__float_as_uint(vreg[j][c]) & 0x7f800000u) == 0x7f800000u;
+        }
+        __syncthreads();  // the previous tile has been read
+        store_tile();
+        __syncthreads();
+        if (kt + 1 < nkt) load_tile(kt + 1);
+
+        // key blocks in pairs (keys kv0 + 32p .. + 31); a pair past the
+        // sequence or wholly above the wave's diagonal is skipped
+        const int lim = min(seq, causal ? wrow0 + 16 : seq);  // first masked key, at most
+        const int np = wrow0 >= seq ? 0 : min(2, (lim - kv0 + 31) / 32);
+        __builtin_amdgcn_s_setprio(0);
+        f32x4 sc[4];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            if (p >= np) break;
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                // eight partial sums a key block: rounding chains of D / 32
+                // MFMAs (no longer than prefill_row's lane sums and tree),
+                // and 8 independent MFMA chains
+                f32x4 part[2][4];
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) part[x][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                const float* kp = ks + (32 * p + 16 * kk + r) * kPitch + 4 * g;
+#pragma unroll
+                for (int j = 0; j < kJ; ++j) {
+                    const f32x4 kf = *reinterpret_cast<const f32x4*>(kp + 16 * j);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        part[j & 1][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            kf[c], qf[j][c], part[j & 1][c], 0, 0, 0);
+                }
+                sc[2 * p + kk] = ((part[0][0] + part[0][1]) + (part[0][2] + part[0][3])) +
+                                 ((part[1][0] + part[1][1]) + (part[1][2] + part[1][3]));
+            }
+        }
+        __builtin_amdgcn_s_setprio(1);
+        if (np == 0) continue;
+        if (np < 2) {
+            const float ni = -INFINITY;
+            sc[2] = sc[3] = f32x4{ni, ni, ni, ni};
+        }
+        if ((causal && kv0 + kFT - 1 > wrow0) || kv0 + kFT > seq) {
+            const int last = causal ? min(seq - 1, wrow0 + r) : seq - 1;
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (kv0 + 16 * kb + 4 * g + i > last) sc[kb][i] = -INFINITY;
+        }
+        // online softmax on raw scores, the running maximum moved only by
+        // more than kLazy (log2 domain), as in attn_prefill_mfma
+        float mt = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mt = fmaxf(mt, sc[kb][i]);
+        mt = max4_rows(mt);
+        const bool upd = mt > m_run + lazy_raw;
+        const float m_new = upd ? mt : m_run;
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * scale_log2);
+        m_run = m_new;
+        f32x4 ps = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                // 2^(d c), the product's rounding error put back to first
+                // order: 2^(t + e) = 2^t (1 + e ln 2)
+                const float d = sc[kb][i] - m_use;
+                const float t = d * scale_log2;
+                const float e = fmaf(d, lo_ln2, kLn2 * fmaf(d, scale_log2, -t));
+                const float p2 = __builtin_amdgcn_exp2f(t);
+                sc[kb][i] = p2 > 0.f ? fmaf(p2, e, p2) : p2;
+            }
+            ps += sc[kb];
+        }
+        l_run = l_run * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
+        if (__builtin_amdgcn_ballot_w64(upd)) {
+#pragma unroll
+            for (int hh = 0; hh < kH; ++hh)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) o[hh][c] *= alpha;
+        }
+        __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            if (p >= np) break;
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float* vp = vs + (32 * p + 16 * kk + 4 * g + i) * D + 4 * r;
+#pragma unroll
+                    for (int hh = 0; hh < kH; ++hh) {
+                        const f32x4 vv = *reinterpret_cast<const f32x4*>(vp + 64 * hh);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+                            o[hh][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                vv[c], sc[2 * p + kk][i], o[hh][c], 0, 0, 0);
+                    }
+                }
+        }
+        __builtin_amdgcn_s_setprio(1);
+    }
+
+    float* oh = out + (size_t)bh * seq * D;
+    if (__syncthreads_or(bad)) {
+        for (int row = q0 + wave; row < min(q0 + kFT, seq); row += 4)
+            prefill_row<float>(qh + (size_t)row * D, kh, vh, oh + (size_t)row * D, row + 1, D,
+                               scale, lane);
+        return;
+    }
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    if (wrow0 + r < seq) {
+        float* orow = oh + (size_t)(wrow0 + r) * D + 16 * g;
+#pragma unroll
+        for (int hh = 0; hh < kH; ++hh)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *reinterpret_cast<f32x4*>(orow + 64 * hh + 4 * i) =
+                    f32x4{o[hh][0][i] / l_run, o[hh][1][i] / l_run, o[hh][2][i] / l_run,
+                          o[hh][3][i] / l_run};
+    }
 }
 
 template <typename T>
@@ -581,9 +845,23 @@ void prefill_run(const T* q, const T* k, const T* v, T* out, int batch, int hq, 
     if (batch == 0 || seq == 0) return;  // nothing to compute
     if (!q || !k || !v || !out) inval("attention prefill: null operand");
     const float scale = 1.0f / sqrtf((float)dim);
-    if constexpr (!std::is_same<T, float>::value) {
-        const bool aligned = ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 == 0;
-        if ((dim == 64 || dim == 128) && aligned && !tune(Tune::PrefillForceGeneric, 0)) {
+    const bool aligned = ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 == 0;
+    const bool mfma = (dim == 64 || dim == 128) && aligned && !tune(Tune::PrefillForceGeneric, 0);
+    if constexpr (std::is_same<T, float>::value) {
+        if (mfma) {
+            const long long grid = (long long)batch * hq * ((seq + kFT - 1) / kFT);
+            if (grid > 0x7fffffffLL) inval("attention prefill problem too large for one launch");
+            if (dim == 128)
+                attn_prefill_f32<128><<<(unsigned)grid, 256, 0, s>>>(q, k, v, out, batch, hq, hkv,
+                                                                     seq, causal ? 1 : 0, scale);
+            else
+                attn_prefill_f32<64><<<(unsigned)grid, 256, 0, s>>>(q, k, v, out, batch, hq, hkv,
+                                                                    seq, causal ? 1 : 0, scale);
+            launch_check("attention prefill kernel launch");
+            return;
+        }
+    } else {
+        if (mfma) {
             const long long nqt = (seq + kPQ - 1) / kPQ;
             const long long grid = (long long)batch * hq * nqt;
             if (grid > 0x7fffffffLL) inval("attention prefill problem too large for one launch");

@@ -179,6 +179,51 @@ def test_prefill_f32_generic(b, hq, hkv, s, d, causal):
     np.testing.assert_allclose(staged, out.cpu().numpy(), rtol=0, atol=0)
 
 
+def _nan_equal(a, b):
+    return np.testing.assert_allclose(a.cpu().numpy(), b.cpu().numpy(), rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("s", [1, 15, 16, 17, 63, 64, 65, 96, 129, 300])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_f32_mfma_matches_oracle(d, s, causal, tuning):
+    # S around the 16-row wave, the 32-key pair and the 64-row / key tile;
+    # 8 heads (the XCD order) and 6 (no multiple of 8 with batch 1). The
+    # bar of the float32 tests above; a view off 16-byte alignment and the
+    # forced general kernel give the same values at it.
+    rng = np.random.default_rng(s * 10 + d + int(causal))
+    for b, hq, hkv in ((2, 4, 2), (1, 6, 3)):
+        q, k, v = _inputs(rng, b, hq, hkv, s, d, torch.float32)
+        out = ft.attention_prefill(q, k, v, causal=causal)
+        ref = oracle.attention_prefill(q.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), causal)
+        np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=1e-4, atol=1e-5)
+    shifted = torch.empty(q.numel() + 1, device=DEV)[1:].view_as(q).copy_(q)
+    _nan_equal(ft.attention_prefill(shifted, k, v, causal=causal), out)
+    tuning("FT_PREFILL_FORCE_GENERIC", 1)
+    _nan_equal(ft.attention_prefill(q, k, v, causal=causal), out)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("what", ["inf", "nan", "k"])
+def test_prefill_f32_keys_not_attended_do_not_matter(d, what, tuning):
+    # rows before a key that is not finite (a padded prompt's tail) stay as
+    # they are; the rows that attend it agree with the general kernel
+    rng = np.random.default_rng(d)
+    q, k, v = _inputs(rng, 1, 8, 2, 150, d, torch.float32)
+    clean = ft.attention_prefill(q, k, v)
+    for key in (70, 128, 149):
+        k2, v2 = k.clone(), v.clone()
+        if what == "k":
+            k2[:, :, key:] = float("nan")
+        else:
+            v2[:, :, key:, 3] = float(what)
+        out = ft.attention_prefill(q, k2, v2)
+        _nan_equal(out[:, :, :key], clean[:, :, :key])
+        tuning("FT_PREFILL_FORCE_GENERIC", 1)
+        _nan_equal(out, ft.attention_prefill(q, k2, v2))
+        tuning.clear("FT_PREFILL_FORCE_GENERIC")
+
+
 @pytest.mark.parametrize("dt", HALF)
 @pytest.mark.parametrize("d", [36, 48, 96, 112])
 def test_prefill_half_generic_dims(dt, d):
