@@ -464,7 +464,7 @@ def attention_decode_paged_append(q, k_pool, v_pool, block_table, k_new, v_new, 
     """One decode step over a paged cache: ``kv_append_paged(k_pool, v_pool,
     block_table, k_new, v_new, lens)`` then ``attention_decode_paged(q,
     k_pool, v_pool, block_table, lens + 1)``, in one call (lens is not
-    modified). GPU tensors only. For bf16 / fp16 with D = 128 the decode
+    modified). GPU tensors only. For bf16 / fp16 with D = 64 or 128 the decode
     kernel attends the cached tokens and its combine kernel folds the fresh token into each row's log-sum-exp merge
     (in float32: the output equals the two ops' within the attention
     tolerance) and writes it into the pools (bit for bit), one launch

@@ -15,12 +15,15 @@
 // row's partials with the log-sum-exp rule and divides by l. len == 0 rows
 // produce zeros (reference attention.cu:1349-1350).
 //
-// Two kernel families:
+// Kernel families:
 //   attn_decode_stream bf16/fp16 storage, D == 128, G <= 16: QK^T and PV on
 //     + attn_combine_  the matrix cores (v_mfma_f32_16x16x32_{bf16,f16});
 //       stream         every K/V byte is read once, straight into the MFMA
 //                      operand layout with 16-byte loads, double-buffered;
 //                      equal token segments per workgroup (stream split).
+//   attn_decode_wide   the same split for bf16/fp16 with D == 64 and float32
+//     + attn_combine_  with D == 64 or 128 (v_mfma_f32_16x16x4_f32), G <= 16.
+//       stream
 //   attn_chunk_generic any storage type, D % 4 == 0 <= 512, any G: VALU
 //     + attn_combine   dot products, chunk scores staged in LDS; the grid
 //                      covers the cache capacity in fixed chunks.
@@ -318,6 +321,13 @@ constexpr int kStreamScanRows = 2048;        // sequences per launch (LDS prefix
 // tokens (fp16, HIP-graph replays) takes 24.6 us at 1024 (128 segments),
 // 20.0 us at 512, 21.3 us at 256.
 constexpr int kStreamMinSeg = 512;
+// A call too small to give every CU that many takes shorter segments, one
+// per CU, down to this (bf16, 4 rows of 10-2000 tokens, 8 kv heads: 16.4 us
+// against 23.3 with 512 tokens) - or to half of it where those still leave
+// CUs idle (fp16, D = 64, 4 rows of 10-200 tokens: 14.3 against 17.5 us; four
+// rows of 128-1024 tokens, which do not, are better off at 128: 11.7 against
+// 12.7 us with 64).
+constexpr int kStreamLowSeg = 128;
 
 // Rows of equal length, each at least this long, take one segment per CU
 // instead of two when the host launched the default two per CU (the
@@ -380,9 +390,103 @@ __device__ __forceinline__ long long uniform64(long long x) {
     return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
-__device__ __forceinline__ long long stream_seg_len(long long total, int nseg, int min_seg) {
+// Tokens per segment: `total` over nseg segments, at least min_seg of them -
+// or, when that would leave CUs without a segment (cus > 0: their count), as
+// many as give each CU one, down to low_seg (half of it where even those
+// leave CUs without one: short rows, where a segment holds several pieces).
+__device__ __forceinline__ long long stream_seg_len(long long total, int nseg, int min_seg,
+                                                    int low_seg, int cus) {
     const long long s = (total + nseg - 1) / nseg;
-    return s < min_seg ? (long long)min_seg : s;
+    long long least = min_seg;
+    if (cus > 0) {
+        const long long low = total <= (long long)cus * (low_seg / 2) ? low_seg / 2 : low_seg;
+        least = max(low, min(least, (total + cus - 1) / cus));
+    }
+    return s < least ? least : s;
+}
+
+// Segments of this launch: the grid, or half of it for long rows of equal
+// length (kStreamUniformLong; cus > 0 says the library chose the grid).
+__device__ __forceinline__ int stream_segments(const int* s_mm, int cus) {
+    int nseg = (int)gridDim.x;
+    if (cus > 0 && nseg > cus && s_mm[0] == s_mm[1] && s_mm[0] >= kStreamUniformLong) nseg = (nseg + 1) >> 1;
+    return __builtin_amdgcn_readfirstlane(nseg);
+}
+
+// A flat position's place: row (b, kv) and the tokens [t0, t0 + n) of it
+// that lie before seg_hi. Everything is wave-uniform.
+struct StreamPiece {
+    int b, kv, row, t0, n;
+    bool whole;       // the row's every token
+    long long next;   // the flat position behind the piece
+};
+
+__device__ __forceinline__ StreamPiece stream_piece(const long long* s_pref, int batch, int hkv,
+                                                    long long pos, long long seg_hi) {
+    int lo = 0, hi = batch - 1;  // last sequence starting at or before pos
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (uniform64(s_pref[mid]) * hkv <= pos) lo = mid; else hi = mid - 1;
+    }
+    StreamPiece p;
+    p.b = lo;
+    const long long pb = uniform64(s_pref[lo]);
+    const long long base = pb * hkv;
+    const int len = (int)(uniform64(s_pref[lo + 1]) - pb);
+    p.kv = (int)((pos - base) / len);
+    p.t0 = (int)(pos - base - (long long)p.kv * len);
+    p.next = min(seg_hi, base + (long long)(p.kv + 1) * len);
+    p.n = (int)(p.next - pos);
+    p.whole = p.t0 == 0 && p.n == len;
+    p.row = lo * hkv + p.kv;
+    return p;
+}
+
+// acc / l. Half storage rounds the quotient anyway: one reciprocal.
+template <typename T>
+__device__ __forceinline__ float4 over_sum(float4 a, float l) {
+    if constexpr (std::is_same<T, float>::value)
+        return make_float4(a.x / l, a.y / l, a.z / l, a.w / l);
+    const float inv = 1.0f / l;
+    return make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+}
+
+// The end of a piece: the 4 waves' (m, l, acc[head][D]) in LDS (rows of D + 4
+// floats) folded for each of the group's heads, then the normalised row
+// stored (a whole row, unless every piece leaves its partial) or the partial.
+template <typename T, int D, bool NEW>
+__device__ __forceinline__ void stream_store(const float (&s_acc)[4][16][D + 4],
+                                             const float (&s_m)[4][16],
+                                             const float (&s_l)[4][16], int tid, int group,
+                                             size_t slot0, bool whole, T* __restrict__ orow,
+                                             float* __restrict__ ws_ml,
+                                             float* __restrict__ ws_acc) {
+    const int nvec = group * (D / 4);
+    for (int idx = tid; idx < nvec; idx += 256) {
+        const int hh = idx / (D / 4);
+        const int d4 = idx - hh * (D / 4);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) mx = fmaxf(mx, s_m[w][hh]);
+        float lsum = 0.0f;
+        float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float wt = exp2f(s_m[w][hh] - mx);
+            lsum += s_l[w][hh] * wt;
+            const float4 a = *reinterpret_cast<const float4*>(&s_acc[w][hh][4 * d4]);
+            o.x += wt * a.x; o.y += wt * a.y; o.z += wt * a.z; o.w += wt * a.w;
+        }
+        if (whole && !NEW) {
+            St<T>::st4(orow + (size_t)hh * D + 4 * d4, over_sum<T>(o, lsum));
+        } else {
+            *reinterpret_cast<float4*>(ws_acc + (slot0 + hh) * D + 4 * d4) = o;
+            if (d4 == 0) {
+                ws_ml[(slot0 + hh) * 2] = mx;
+                ws_ml[(slot0 + hh) * 2 + 1] = lsum;
+            }
+        }
+    }
 }
 
 // The fresh token of the appending decode: ap.k_new / ap.v_new [batch, hkv,
@@ -398,11 +502,10 @@ struct AppendArgs {
 };
 
 // Element offset of row (b, kv)'s cache position t in a pool.
-template <int MODE>
+template <int D, int MODE>
 __device__ __forceinline__ size_t kv_row_offset(const int* table, int b, int kv, int t, int hkv,
                                                 int rows_or_page, int page_shift,
                                                 int tbl_width) {
-    constexpr int D = kMfmaDim;
     if constexpr (MODE == kRowsContig) {
         return ((size_t)(b * hkv + kv) * rows_or_page + t) * D;
     } else {
@@ -423,7 +526,7 @@ void attn_decode_stream(
     float* __restrict__ ws_ml, float* __restrict__ ws_acc,
     long long* __restrict__ pref_out, T* __restrict__ out, int batch, int hq, int hkv,
     int group, int rows_or_page, int page_shift, int tbl_width, int span, float scale_log2,
-    int min_seg, int halve) {
+    int min_seg, int low_seg, int cus) {
     using M = Mfma<T>;
     using V8 = typename M::v8;
     constexpr int D = kMfmaDim;
@@ -441,16 +544,13 @@ void attn_decode_stream(
 
     if (wave == 0) scan_lengths(lens, batch, span, lane, s_pref, s_mm);
     __syncthreads();
-    // segments: the grid, or half of it for long rows of equal length
-    int nseg = (int)gridDim.x;
-    if (halve && s_mm[0] == s_mm[1] && s_mm[0] >= kStreamUniformLong) nseg = (nseg + 1) >> 1;
-    nseg = __builtin_amdgcn_readfirstlane(nseg);
-    if (blockIdx.x == 0) {  // the combine kernel's copy of the prefix and the count
-        for (int i = tid; i <= batch; i += 256) pref_out[i] = s_pref[i];
-        if (tid == 0) pref_out[batch + 1] = nseg;
-    }
+    const int nseg = stream_segments(s_mm, cus);
     const long long total = uniform64(s_pref[batch]) * hkv;
-    const long long S = stream_seg_len(total, nseg, min_seg);
+    const long long S = stream_seg_len(total, nseg, min_seg, low_seg, cus);
+    if (blockIdx.x == 0) {  // the combine kernel's copy of the prefix, and S
+        for (int i = tid; i <= batch; i += 256) pref_out[i] = s_pref[i];
+        if (tid == 0) pref_out[batch + 1] = S;
+    }
     const long long seg_lo = (long long)blockIdx.x * S;
     if (seg_lo >= total) return;
     const long long seg_hi = min(seg_lo + S, total);
@@ -466,22 +566,8 @@ void attn_decode_stream(
     long long pos = seg_lo;
     while (pos < seg_hi) {
         // ---- locate the piece: row (b, kv), tokens [t0, t0 + n) ------------
-        int lo = 0, hi = batch - 1;  // last sequence starting at or before pos
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (uniform64(s_pref[mid]) * hkv <= pos) lo = mid; else hi = mid - 1;
-        }
-        const int b = lo;
-        const long long pb = uniform64(s_pref[b]);
-        const long long base = pb * hkv;
-        const int len = (int)(uniform64(s_pref[b + 1]) - pb);
-        const int kv = (int)((pos - base) / len);
-        const int t0 = (int)(pos - base - (long long)kv * len);
-        const long long row_end = base + (long long)(kv + 1) * len;
-        const long long piece_hi = min(seg_hi, row_end);
-        const int n = (int)(piece_hi - pos);
-        const bool whole = (t0 == 0 && n == len);
-        const int row = b * hkv + kv;
+        const StreamPiece pc = stream_piece(s_pref, batch, hkv, pos, seg_hi);
+        const int b = pc.b, kv = pc.kv, row = pc.row, t0 = pc.t0, n = pc.n;
         const int* trow = PAGED ? table + (size_t)b * tbl_width : nullptr;
         // B operand of the score MFMAs: Q[head r][32j + 8g .. +7]
         V8 qb[4];
@@ -681,72 +767,412 @@ void attn_decode_stream(
             for (int i = 0; i < 4; ++i) s_acc[wave][r][16 * nn + 4 * g + i] = acc[nn][i];
         __syncthreads();
 
-        const int nvec = group * (D / 4);
-        const size_t slot0 = ((size_t)blockIdx.x + row) * group;
-        T* const orow = out + ((size_t)b * hq + (size_t)kv * group) * D;
-        for (int idx = tid; idx < nvec; idx += 256) {
-            const int hh = idx / (D / 4);
-            const int d4 = idx - hh * (D / 4);
-            float mx = -INFINITY;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) mx = fmaxf(mx, s_m[w][hh]);
-            float lsum = 0.0f;
-            float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const float wt = exp2f(s_m[w][hh] - mx);
-                lsum += s_l[w][hh] * wt;
-                const float4 a = *reinterpret_cast<const float4*>(&s_acc[w][hh][4 * d4]);
-                o.x += wt * a.x; o.y += wt * a.y; o.z += wt * a.z; o.w += wt * a.w;
-            }
-            if (whole && !NEW) {
-                const float inv = 1.0f / lsum;
-                St<T>::st4(orow + (size_t)hh * D + 4 * d4,
-                           make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv));
-            } else {
-                *reinterpret_cast<float4*>(ws_acc + (slot0 + hh) * D + 4 * d4) = o;
-                if (d4 == 0) {
-                    ws_ml[(slot0 + hh) * 2] = mx;
-                    ws_ml[(slot0 + hh) * 2 + 1] = lsum;
-                }
-            }
-        }
+        stream_store<T, D, NEW>(s_acc, s_m, s_l, tid, group, ((size_t)blockIdx.x + row) * group,
+                                pc.whole, out + ((size_t)b * hq + (size_t)kv * group) * D, ws_ml,
+                                ws_acc);
         __syncthreads();  // LDS is reused by the next piece
-        pos = piece_hi;
+        pos = pc.next;
     }
 }
 
 // ---------------------------------------------------------------------------
-// combine for attn_decode_stream, one wave per (b, q head). Row (b, kv)
+// The stream decode for the other row sizes: bf16 / fp16 with D = 64, float32
+// with D = 64 or 128 (attn_decode_stream keeps half storage with D = 128,
+// whose main loop it is tuned around). Same work split, pieces, partials and
+// memory pipeline: K / V of two steps in registers, the step after next's
+// loads issued before a step is computed, whole 128-byte lines per load
+// instruction, non-temporal.
+//
+// Half storage, D = 64: 32-token steps. K and V go through the wave's LDS
+// staging (32 rows x 128 B each; chunk c of row w at c ^ ((w >> 1) & 7), so
+// the 16 lanes of a write - two rows - and of a fragment read - 16 rows, one
+// chunk - hit 16 different 16-byte bank groups), K into the score MFMAs' A
+// operand, V through ds_read_b64_tr_b16 straight into the PV product's (no
+// transposing MFMAs): source lane s of group g addresses V row 4g + s / 4
+// (+ 16), columns 16 db + 4 (s % 4) .. + 3, and lane (d, g) gets keys 4g + i.
+//
+// float32: 16-token steps on v_mfma_f32_16x16x4_f32 (A[r][g], B[g][r],
+// C[4g+i][r]), every product and sum float32. K through the staging (chunk c
+// of row w at c ^ w): lane (r, g) reads K[tok r][16j + 4g .. +3] and feeds 4
+// MFMAs, k slot g being dim 16j + 4g + c; eight partial sums keep the
+// rounding chains short. V needs no staging: MFMA i of the PV product takes
+// the weight the lane holds for token 4g + i as B, so lane (r, g) loads
+// V[tok 4g + i][64h + 4r .. +3] (256 contiguous bytes per 16 lanes) as A,
+// output row r of MFMA (h, c) being dim 64h + 4r + c.
+//
+// Tokens past the piece weigh 0 and their V is set to 0, so a V value that is
+// not finite reaches only the rows that attend it.
+//
+// What bounds it: HBM, as attn_decode_stream. At one 16 x 16 tile per 16
+// tokens the float32 products take 1/3 of the matrix rate at 6 TB/s.
+// Measured against attn_chunk_generic + attn_combine, which ran these shapes:
+// float32 32 / 8 heads, D = 128, one row of 16384 tokens 109 -> 32 us (4.1
+// TB/s); 16 rows of 100-8000 tokens, paged, 447 -> 117 us (4.6 TB/s); bf16,
+// D = 64, 64 such rows 1050 -> 110 us (4.7 TB/s); 4 rows of 128-1024 tokens,
+// bf16, D = 64, 26.8 -> 12.3 us (graph replays). Error against 64 bits, f32:
+// 2.0e-7 where the general kernel has 2.7e-7 (16384 tokens).
+// ---------------------------------------------------------------------------
+template <typename T, int D>
+struct WideStep {
+    static constexpr bool kF32 = std::is_same<T, float>::value;
+    static constexpr int kTok = kF32 ? 16 : 32;              // tokens per step
+    static constexpr int kRowLanes = D * (int)sizeof(T) / 16;  // lanes per row and load
+    static constexpr int kRows = 64 / kRowLanes;             // rows per load instruction
+    static constexpr int kLoads = kTok / kRows;              // K (and V) loads per step
+    static constexpr int kTiles = kTok / 16;                 // 16-token tiles
+    static constexpr int kStage = kTok * D * (int)sizeof(T);   // staged bytes of K (or V)
+    static constexpr int kWave = kF32 ? kStage : 2 * kStage;
+    static constexpr int kAcc = 16 * (D + 4) * 4;            // a wave's merge rows
+    // workgroups per CU: two steps of float32 rows with D = 128 need more than
+    // half the registers (two per CU spill 28: 38 against 31 us for one row
+    // of 16384 tokens)
+    static constexpr int kOccupancy = kF32 && D == 128 ? 1 : 2;
+};
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+template <typename T, int D, int MODE, bool NEW>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(WideStep<T, D>::kOccupancy, WideStep<T, D>::kOccupancy)))
+void attn_decode_wide(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
+    const int* __restrict__ table, const int* __restrict__ lens,
+    float* __restrict__ ws_ml, float* __restrict__ ws_acc,
+    long long* __restrict__ pref_out, T* __restrict__ out, int batch, int hq, int hkv,
+    int group, int rows_or_page, int page_shift, int tbl_width, int span, float scale_log2,
+    int min_seg, int low_seg, int cus) {
+    using W = WideStep<T, D>;
+    constexpr bool F32 = W::kF32;
+    constexpr bool PAGED = MODE != kRowsContig;
+    constexpr int kTok = W::kTok, kRows = W::kRows, kRowLanes = W::kRowLanes;
+    constexpr int kElems = 16 / (int)sizeof(T);  // elements per 16-byte chunk
+    // the merge rows of the 4 waves alias their staging
+    constexpr int kMerge = 4 * W::kAcc;
+    constexpr int kStaging = 4 * W::kWave;
+    __shared__ __attribute__((aligned(16))) char s_raw[kMerge > kStaging ? kMerge : kStaging];
+    float (&s_acc)[4][16][D + 4] = *reinterpret_cast<float (*)[4][16][D + 4]>(s_raw);
+    __shared__ float s_m[4][16], s_l[4][16];
+    __shared__ long long s_pref[kStreamScanRows + 1];
+    __shared__ int s_mm[2];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+
+    if (wave == 0) scan_lengths(lens, batch, span, lane, s_pref, s_mm);
+    __syncthreads();
+    const int nseg = stream_segments(s_mm, cus);
+    const long long total = uniform64(s_pref[batch]) * hkv;
+    const long long S = stream_seg_len(total, nseg, min_seg, low_seg, cus);
+    if (blockIdx.x == 0) {  // the combine kernel's copy of the prefix, and S
+        for (int i = tid; i <= batch; i += 256) pref_out[i] = s_pref[i];
+        if (tid == 0) pref_out[batch + 1] = S;
+    }
+    const long long seg_lo = (long long)blockIdx.x * S;
+    if (seg_lo >= total) return;
+    const long long seg_hi = min(seg_lo + S, total);
+
+    char* const stg = s_raw + wave * W::kWave;
+
+    long long pos = seg_lo;
+    while (pos < seg_hi) {
+        const StreamPiece pc = stream_piece(s_pref, batch, hkv, pos, seg_hi);
+        const int kv = pc.kv, row = pc.row, t0 = pc.t0, n = pc.n;
+        const int* trow = PAGED ? table + (size_t)pc.b * tbl_width : nullptr;
+        // B operand of the score MFMAs, 16-byte chunk 4j + g of head r
+        constexpr int kQ = D / (4 * kElems);
+        u32x4 qb[kQ];
+        {
+            const bool ok = r < group;
+            const T* qrow = q + ((size_t)pc.b * hq + (size_t)kv * group + (ok ? r : 0)) * D;
+#pragma unroll
+            for (int j = 0; j < kQ; ++j) {
+                const u32x4 x = *reinterpret_cast<const u32x4*>(qrow + kElems * (4 * j + g));
+                const u32x4 z = {0u, 0u, 0u, 0u};
+                qb[j] = ok ? x : z;
+            }
+        }
+
+        f32x4 acc[D / 16];
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float m_run = -INFINITY, l_run = 0.0f;
+
+        auto tbl_load = [&](int st, int (&e)[W::kTiles]) {
+            if constexpr (PAGED) {
+#pragma unroll
+                for (int h = 0; h < W::kTiles; ++h) {
+                    const int t = t0 + min(st * kTok + 16 * h + r, n - 1);
+                    e[h] = trow[MODE == kRowsPagedPow2 ? (t >> page_shift) : (t / rows_or_page)];
+                }
+            }
+        };
+        // element offset of step token rho (a row of the cache); past the
+        // piece: its last token
+        auto row_at = [&](int st, const int (&e)[W::kTiles], int h, int rho) {
+            const int t = t0 + min(st * kTok + 16 * h + rho, n - 1);
+            if constexpr (MODE == kRowsContig) {
+                return ((size_t)row * rows_or_page + t) * D;
+            } else {
+                const int ent = __shfl(e[h], rho, 64);
+                const int in_pg = MODE == kRowsPagedPow2 ? (t & (rows_or_page - 1))
+                                                         : (t % rows_or_page);
+                return (((size_t)ent * hkv + kv) * rows_or_page + in_pg) * D;
+            }
+        };
+        auto kv_load = [&](int st, const int (&e)[W::kTiles], u32x4 (&kt)[W::kLoads],
+                           u32x4 (&vt)[W::kLoads]) {
+#pragma unroll
+            for (int p = 0; p < W::kLoads; ++p) {
+                const int h = p * kRows / 16;
+                const size_t off = row_at(st, e, h, p * kRows - 16 * h + lane / kRowLanes) +
+                                   kElems * (lane % kRowLanes);
+                kt[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(k + off));
+                if constexpr (!F32)
+                    vt[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(v + off));
+            }
+            if constexpr (F32) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const size_t off = row_at(st, e, 0, 4 * g + i) + 4 * r;
+#pragma unroll
+                    for (int hh = 0; hh < D / 64; ++hh)
+                        vt[i * (D / 64) + hh] = __builtin_nontemporal_load(
+                            reinterpret_cast<const u32x4*>(v + off + 64 * hh));
+                }
+            }
+        };
+        auto compute_step = [&](int st, const u32x4 (&kin)[W::kLoads], u32x4 (&vin)[W::kLoads]) {
+            const int tb = st * kTok;
+            const u32x4 z4 = {0u, 0u, 0u, 0u};
+            if (tb + kTok > n) {  // the piece's end: V of the tokens past it
+#pragma unroll
+                for (int p = 0; p < W::kLoads; ++p) {
+                    const int w = F32 ? 4 * g + p / (D / 64) : p * kRows + lane / kRowLanes;
+                    if (tb + w >= n) vin[p] = z4;
+                }
+            }
+            // swizzled byte offset of 16-byte chunk c of staged row w
+            auto at = [&](int w, int c) {
+                return w * (D * (int)sizeof(T)) + 16 * (c ^ (F32 ? w : (w >> 1) & 7));
+            };
+            wave_lds_order();  // the previous step's reads come first
+#pragma unroll
+            for (int p = 0; p < W::kLoads; ++p) {
+                const int w = p * kRows + lane / kRowLanes;
+                *reinterpret_cast<u32x4*>(stg + at(w, lane % kRowLanes)) = kin[p];
+                if constexpr (!F32)
+                    *reinterpret_cast<u32x4*>(stg + W::kStage + at(w, lane % kRowLanes)) = vin[p];
+            }
+            wave_lds_order();
+            f32x4 s[W::kTiles];
+            if constexpr (F32) {
+                // 4 partial sums over every 32 dims
+#pragma unroll
+                for (int x = 0; x < kQ / 2; ++x) {
+                    f32x4 part[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) part[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int j = 2 * x; j < 2 * x + 2; ++j) {
+                        const f32x4 kf = *reinterpret_cast<const f32x4*>(stg + at(r, 4 * j + g));
+                        const f32x4 qf = __builtin_bit_cast(f32x4, qb[j]);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+                            part[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c], qf[c], part[c],
+                                                                           0, 0, 0);
+                    }
+                    const f32x4 sum = (part[0] + part[1]) + (part[2] + part[3]);
+                    s[0] = x ? s[0] + sum : sum;
+                }
+            } else {
+                using V8 = typename Mfma<T>::v8;
+#pragma unroll
+                for (int h = 0; h < W::kTiles; ++h) {
+                    s[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int j = 0; j < kQ; ++j)
+                        s[h] = Mfma<T>::mma(
+                            *reinterpret_cast<const V8*>(stg + at(16 * h + r, 4 * j + g)),
+                            __builtin_bit_cast(V8, qb[j]), s[h]);
+                }
+            }
+            float mloc = -INFINITY;
+#pragma unroll
+            for (int h = 0; h < W::kTiles; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (tb + 16 * h + 4 * g + i >= n) s[h][i] = -INFINITY;
+                    mloc = fmaxf(mloc, s[h][i]);
+                }
+            // m in log2 units (scale_log2 > 0 commutes with max); the weights
+            // 2^(s scale - m) round once
+            const float m_new = fmaxf(m_run, max4_rows(mloc) * scale_log2);
+            const float m_use = m_new == -INFINITY ? 0.f : m_new;
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+            m_run = m_new;
+            float psum = 0.0f;
+#pragma unroll
+            for (int h = 0; h < W::kTiles; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[h][i] = __builtin_amdgcn_exp2f(fmaf(s[h][i], scale_log2, -m_use));
+                    psum += s[h][i];
+                }
+            l_run = l_run * alpha + psum;
+            if constexpr (F32) {
+                // the step's own sum first: one rounding a step in acc
+#pragma unroll
+                for (int hh = 0; hh < D / 64; ++hh) {
+                    f32x4 sum[4], odd[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) sum[c] = odd[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const f32x4 vv = __builtin_bit_cast(f32x4, vin[i * (D / 64) + hh]);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            f32x4& x = i & 1 ? odd[c] : sum[c];
+                            x = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[c], s[0][i], x, 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) sum[c] += odd[c];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            acc[4 * hh + c][i] = fmaf(acc[4 * hh + c][i], alpha, sum[c][i]);
+                }
+            } else {
+#pragma unroll
+                for (int nn = 0; nn < D / 16; ++nn) acc[nn] *= alpha;
+                using V8 = typename Mfma<T>::v8;
+                typedef short v4s __attribute__((ext_vector_type(4)));
+                typedef short v8s __attribute__((ext_vector_type(8)));
+                // the weights in parts of T, truncated: all 24 significant
+                // bits (3 bf16) or 22 (2 fp16). No part is 0 unless the weight
+                // is, so every product of a weight and an infinite V value is
+                // that infinity (the general kernel's result)
+                constexpr int kParts = std::is_same<T, bf16>::value ? 3 : 2;
+                V8 pp[kParts];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float p = s[i >> 2][i & 3];
+                    float rest = p;
+#pragma unroll
+                    for (int x = 0; x < kParts; ++x) {
+                        float hi, least;
+                        if constexpr (std::is_same<T, bf16>::value) {
+                            hi = __uint_as_float(__float_as_uint(rest) & 0xffff0000u);
+                            least = 0x1p-126f;
+                        } else {
+                            hi = (float)__builtin_amdgcn_cvt_pkrtz(rest, 0.f)[0];
+                            least = 0x1p-24f;
+                        }
+                        rest -= hi;
+                        pp[x][i] = (T)(x > 0 && p > 0.f ? fmaxf(hi, least) : hi);
+                    }
+                }
+#pragma unroll
+                for (int db = 0; db < D / 16; ++db) {
+                    const int w = 4 * g + (r >> 2);
+                    const int c = 2 * db + ((r & 3) >> 1);
+                    const char* lo_p = stg + W::kStage + at(w, c) + 8 * (r & 1);
+                    const char* hi_p = stg + W::kStage + at(w + 16, c) + 8 * (r & 1);
+                    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) v4s*)(lo_p));
+                    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) v4s*)(hi_p));
+                    const V8 va = __builtin_bit_cast(
+                        V8, v8s{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+#pragma unroll
+                    for (int x = 0; x < kParts; ++x)
+                        acc[db] = Mfma<T>::mma(va, pp[x], acc[db]);
+                }
+            }
+        };
+
+        // ---- stream the piece: two steps per iteration (buffers A, B) ------
+        const int nsteps = (n + kTok - 1) / kTok;
+        const int last = nsteps - 1;
+        int st = wave;
+        if (st < nsteps) {
+            u32x4 ka[W::kLoads], va_[W::kLoads], kb[W::kLoads], vb[W::kLoads];
+            int ea[W::kTiles] = {}, eb[W::kTiles] = {};
+            tbl_load(st, ea);
+            tbl_load(min(st + 4, last), eb);
+            kv_load(st, ea, ka, va_);
+            for (; st + 4 < nsteps; st += 8) {
+                tbl_load(min(st + 8, last), ea);
+                kv_load(st + 4, eb, kb, vb);
+                __builtin_amdgcn_sched_barrier(0);  // the prefetch stays ahead
+                compute_step(st, ka, va_);
+                tbl_load(min(st + 12, last), eb);
+                kv_load(min(st + 8, last), ea, ka, va_);
+                __builtin_amdgcn_sched_barrier(0);
+                compute_step(st + 4, kb, vb);
+            }
+            if (st < nsteps) compute_step(st, ka, va_);
+        }
+
+        // ---- merge the 4 waves, then store the row or the piece's partial --
+        l_run += __shfl_xor(l_run, 16, 64);
+        l_run += __shfl_xor(l_run, 32, 64);
+        // the merge rows may lie in another wave's staging
+        if constexpr (W::kAcc != W::kWave) __syncthreads();
+        if (lane < 16) {
+            s_m[wave][lane] = m_run;
+            s_l[wave][lane] = l_run;
+        }
+#pragma unroll
+        for (int nn = 0; nn < D / 16; ++nn)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                // acc[4h + c][i] of float32: dim 64h + 16g + 4i + c
+                const int d = F32 ? 64 * (nn >> 2) + 16 * g + 4 * i + (nn & 3)
+                                  : 16 * nn + 4 * g + i;
+                s_acc[wave][r][d] = acc[nn][i];
+            }
+        __syncthreads();
+        stream_store<T, D, NEW>(s_acc, s_m, s_l, tid, group, ((size_t)blockIdx.x + row) * group,
+                                pc.whole, out + ((size_t)pc.b * hq + (size_t)kv * group) * D,
+                                ws_ml, ws_acc);
+        __syncthreads();  // LDS is reused by the next piece
+        pos = pc.next;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// combine for attn_decode_stream / attn_decode_wide, one wave per (b, q head). Row (b, kv)
 // spans segments [s_lo, s_hi] of length S; its pieces' partials sit at
 // slots s + row. A row inside one segment was stored by the decode kernel;
 // a row of length 0 is zero-filled here (reference attention.cu:1349-1350).
-// Lanes split into 2 groups of 32 (one float4 column of D = 128 each) that
-// walk alternate pieces; the groups are summed with one xor shuffle.
+// Lanes split into 256 / D groups of D / 4 (one float4 column each) that
+// walk the pieces in turn; the groups are summed with xor shuffles.
 // Returns the head's stored output (as T, widened to f32), columns
-// 4 (lane & 31) .. + 3, in every lane.
+// 4 (lane mod D / 4) .. + 3, in every lane.
 // ---------------------------------------------------------------------------
-template <typename T>
+template <typename T, int D>
 __device__ __forceinline__ float4 combine_head(const float* __restrict__ ws_ml,
                                                const float* __restrict__ ws_acc,
                                                const long long* __restrict__ pref,
                                                T* __restrict__ out, int bh, int batch, int hq,
-                                               int hkv, int group, int min_seg, int lane,
+                                               int hkv, int group, int lane,
                                                bool skip_empty = false) {
-    constexpr int D = kMfmaDim;
     const int b = bh / hq;
     const int h = bh - b * hq;
     const int kv = h / group, gi = h - kv * group;
     T* o = out + (size_t)bh * D;
     const int len = (int)(pref[b + 1] - pref[b]);
-    const int d4 = lane & 31;
+    const int d4 = lane & (D / 4 - 1);
     if (len == 0) {  // (skip_empty: written by the decode kernel)
         if (!skip_empty && lane < D / 4)
             St<T>::st4(o + 4 * lane, make_float4(0.f, 0.f, 0.f, 0.f));
         return make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    // the decode kernel's segment count, after the prefix
-    const long long S = stream_seg_len(pref[batch] * hkv, (int)pref[batch + 1], min_seg);
+    const long long S = pref[batch + 1];  // the decode kernel's segment length
     const long long start = pref[b] * hkv + (long long)kv * len;
     const int s_lo = (int)(start / S), s_hi = (int)((start + len - 1) / S);
     // stored whole by the decode kernel: its stored values, read back here
@@ -764,46 +1190,49 @@ __device__ __forceinline__ float4 combine_head(const float* __restrict__ ws_ml,
     for (int i = lane; i < np; i += 64)
         lsum += ws_ml[slot(i) * 2 + 1] * exp2f(ws_ml[slot(i) * 2] - mx);
     lsum = wave_sum(lsum);
-    const int grp = lane >> 5;
+    const int grp = lane / (D / 4);
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 4
-    for (int i = grp; i < np; i += 2) {
+    for (int i = grp; i < np; i += 256 / D) {
         const size_t sl = slot(i);
         const float wt = exp2f(ws_ml[sl * 2] - mx);
         const float4 x = *reinterpret_cast<const float4*>(ws_acc + sl * D + 4 * d4);
         a.x += wt * x.x; a.y += wt * x.y; a.z += wt * x.z; a.w += wt * x.w;
     }
-    a.x += __shfl_xor(a.x, 32, 64);
-    a.y += __shfl_xor(a.y, 32, 64);
-    a.z += __shfl_xor(a.z, 32, 64);
-    a.w += __shfl_xor(a.w, 32, 64);
-    const float inv = 1.0f / lsum;
-    const float4 ov = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+#pragma unroll
+    for (int o2 = 32; o2 >= D / 4; o2 >>= 1) {
+        a.x += __shfl_xor(a.x, o2, 64);
+        a.y += __shfl_xor(a.y, o2, 64);
+        a.z += __shfl_xor(a.z, o2, 64);
+        a.w += __shfl_xor(a.w, o2, 64);
+    }
+    const float4 ov = over_sum<T>(a, lsum);
     if (grp == 0) St<T>::st4(o + 4 * d4, ov);
     return make_float4((float)(T)ov.x, (float)(T)ov.y, (float)(T)ov.z, (float)(T)ov.w);
 }
 
-// max |v| over a head's 128 stored values (lanes 0-31 hold them all, and
-// lanes 32-63 the same again), in every lane
+// max |v| over a head's D stored values (lanes 0 .. D / 4 - 1 hold them all,
+// the others the same again), in every lane
+template <int D>
 __device__ __forceinline__ float head_absmax(float4 v) {
     float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 #pragma unroll
-    for (int o2 = 16; o2 > 0; o2 >>= 1) m = fmaxf(m, __shfl_xor(m, o2, 64));
+    for (int o2 = D / 8; o2 > 0; o2 >>= 1) m = fmaxf(m, __shfl_xor(m, o2, 64));
     return m;
 }
 
 // AMAX: the max |stored output| of each head into amax[b * hq + h], which
 // the per-tensor quantize of the output folds. skip_empty: rows of length 0
 // were written by the decode kernel (its append form).
-template <typename T, bool AMAX>
+template <typename T, int D, bool AMAX>
 __global__ __launch_bounds__(64) void attn_combine_stream(
     const float* __restrict__ ws_ml, const float* __restrict__ ws_acc,
     const long long* __restrict__ pref, T* __restrict__ out, float* __restrict__ amax,
-    int batch, int hq, int hkv, int group, int min_seg, int skip_empty) {
-    const float4 v = combine_head<T>(ws_ml, ws_acc, pref, out, blockIdx.x, batch, hq, hkv,
-                                     group, min_seg, threadIdx.x, skip_empty != 0);
+    int batch, int hq, int hkv, int group, int skip_empty) {
+    const float4 v = combine_head<T, D>(ws_ml, ws_acc, pref, out, blockIdx.x, batch, hq, hkv,
+                                        group, threadIdx.x, skip_empty != 0);
     if constexpr (AMAX) {
-        const float m = head_absmax(v);
+        const float m = head_absmax<D>(v);
         if (threadIdx.x == 0) amax[blockIdx.x] = m;
     }
 }
@@ -816,23 +1245,22 @@ __global__ __launch_bounds__(64) void attn_combine_stream(
 // decode kernel has finished reading them). A row with no cached token gets
 // v_new alone (softmax weight 1: exactly v_new), or zeros when lens[b] has
 // no room in the row or is negative (kv_append_paged then writes nothing).
-template <typename T, int MODE>
+template <typename T, int D, int MODE>
 __global__ __launch_bounds__(64) void attn_combine_append(
     const float* __restrict__ ws_ml, const float* __restrict__ ws_acc,
     const long long* __restrict__ pref, const int* __restrict__ lens, const T* __restrict__ q,
     AppendArgs<T> ap, const int* __restrict__ table, T* __restrict__ out, int batch, int hq,
-    int hkv, int group, int min_seg, int span, int rows_or_page, int page_shift,
-    int tbl_width, float scale_log2) {
-    constexpr int D = kMfmaDim;
+    int hkv, int group, int span, int rows_or_page, int page_shift, int tbl_width,
+    float scale_log2) {
     const int bh = blockIdx.x, lane = threadIdx.x;
     const int b = bh / hq, h = bh - b * hq;
     const int kv = h / group, gi = h - kv * group;
-    const int d4 = lane & 31;
+    const int d4 = lane & (D / 4 - 1);
     T* o = out + (size_t)bh * D;
     const int len = (int)(pref[b + 1] - pref[b]);
     const int raw = lens[b];
     const bool fresh = raw >= 0 && raw < span;  // then raw == len
-    // the fresh token: lane d4 takes dims 4 d4 .. + 3 (lanes 32-63 again)
+    // the fresh token: lane d4 takes dims 4 d4 .. + 3 (the other lanes again)
     float sv = -INFINITY;
     float4 vn = make_float4(0.f, 0.f, 0.f, 0.f);
     if (fresh) {
@@ -845,10 +1273,10 @@ __global__ __launch_bounds__(64) void attn_combine_append(
         dot = fmaf(qq.z, kk.z, dot);
         dot = fmaf(qq.w, kk.w, dot);
 #pragma unroll
-        for (int o2 = 16; o2 > 0; o2 >>= 1) dot += __shfl_xor(dot, o2, 64);
+        for (int o2 = D / 8; o2 > 0; o2 >>= 1) dot += __shfl_xor(dot, o2, 64);
         sv = dot * scale_log2;
-        if (gi == 0 && lane < 32) {
-            const size_t dst = kv_row_offset<MODE>(table, b, kv, raw, hkv, rows_or_page,
+        if (gi == 0 && lane < D / 4) {
+            const size_t dst = kv_row_offset<D, MODE>(table, b, kv, raw, hkv, rows_or_page,
                                                    page_shift, tbl_width) + 4 * d4;
             St<T>::st4(ap.k_pool + dst, kk);
             St<T>::st4(ap.v_pool + dst, vn);
@@ -856,7 +1284,7 @@ __global__ __launch_bounds__(64) void attn_combine_append(
     }
     int s_lo = 0, np = 0;
     if (len > 0) {
-        const long long S = stream_seg_len(pref[batch] * hkv, (int)pref[batch + 1], min_seg);
+        const long long S = pref[batch + 1];  // the decode kernel's segment length
         const long long start = pref[b] * hkv + (long long)kv * len;
         s_lo = (int)(start / S);
         np = (int)((start + len - 1) / S) - s_lo + 1;
@@ -876,19 +1304,22 @@ __global__ __launch_bounds__(64) void attn_combine_append(
     lsum = wave_sum(lsum);
     const float pn = fresh ? exp2f(sv - mx) : 0.0f;
     lsum += pn;
-    const int grp = lane >> 5;
+    const int grp = lane / (D / 4);
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 4
-    for (int i = grp; i < np; i += 2) {
+    for (int i = grp; i < np; i += 256 / D) {
         const size_t sl = slot(i);
         const float wt = exp2f(ws_ml[sl * 2] - mx);
         const float4 x = *reinterpret_cast<const float4*>(ws_acc + sl * D + 4 * d4);
         a.x += wt * x.x; a.y += wt * x.y; a.z += wt * x.z; a.w += wt * x.w;
     }
-    a.x += __shfl_xor(a.x, 32, 64);
-    a.y += __shfl_xor(a.y, 32, 64);
-    a.z += __shfl_xor(a.z, 32, 64);
-    a.w += __shfl_xor(a.w, 32, 64);
+#pragma unroll
+    for (int o2 = 32; o2 >= D / 4; o2 >>= 1) {
+        a.x += __shfl_xor(a.x, o2, 64);
+        a.y += __shfl_xor(a.y, o2, 64);
+        a.z += __shfl_xor(a.z, o2, 64);
+        a.w += __shfl_xor(a.w, o2, 64);
+    }
     a.x += pn * vn.x; a.y += pn * vn.y; a.z += pn * vn.z; a.w += pn * vn.w;
     const float inv = 1.0f / lsum;
     if (grp == 0) St<T>::st4(o + 4 * d4, make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv));
@@ -905,22 +1336,20 @@ __global__ __launch_bounds__(64) void attn_combine_append(
 // with 8 waves and 437.0-437.2 with 4, same box).
 constexpr int kCqWaves = 16;
 
-template <typename T>
+template <typename T, int D>
 __global__ __launch_bounds__(64 * kCqWaves) void attn_combine_quant(
     const float* __restrict__ ws_ml, const float* __restrict__ ws_acc,
     const long long* __restrict__ pref, T* __restrict__ out, signed char* __restrict__ q,
-    float* __restrict__ scale_out, int batch, int hq, int hkv, int group, int min_seg,
-    GridMax gm) {
+    float* __restrict__ scale_out, int batch, int hq, int hkv, int group, GridMax gm) {
     __shared__ float red[kCqWaves];
-    constexpr int D = kMfmaDim;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int bh = blockIdx.x * kCqWaves + wave;
     const bool live = bh < batch * hq;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (live)
-        v = combine_head<T>(ws_ml, ws_acc, pref, out, bh, batch, hq, hkv, group, min_seg, lane);
-    float m = block_max<64 * kCqWaves>(live ? head_absmax(v) : 0.0f, red);
+        v = combine_head<T, D>(ws_ml, ws_acc, pref, out, bh, batch, hq, hkv, group, lane);
+    float m = block_max<64 * kCqWaves>(live ? head_absmax<D>(v) : 0.0f, red);
     m = grid_max<64 * kCqWaves>(gm, m, red);
     const float scale = make_scale(m);
     const float inv_s = 1.0f / scale;
@@ -1037,37 +1466,52 @@ void launch_combine(const float* ws_ml, const float* ws_acc, const int* lens,
 // ---------------------------------------------------------------------------
 // launcher
 // ---------------------------------------------------------------------------
+// The stream kernels' shapes: D = 64 or 128, G <= 16, 16-byte alignment.
 template <typename T>
-bool mfma_eligible(const T* q, const T* k, const T* v, int group, int dim) {
-    if (std::is_same<T, float>::value) return false;
-    if (dim != kMfmaDim || group > 16) return false;
+bool stream_eligible(const T* q, const T* k, const T* v, int group, int dim) {
+    if ((dim != 64 && dim != kMfmaDim) || group > 16) return false;
     return ((uintptr_t)q % 16 == 0) && ((uintptr_t)k % 16 == 0) &&
            ((uintptr_t)v % 16 == 0);
 }
 
-// attn_decode_stream in the row mode of the layout (paged with a power-of-2
-// page, paged with any page, contiguous).
-// fresh: the appending decode's form (NEW).
-template <typename T>
+// attn_decode_stream (half storage, D = 128) or attn_decode_wide in the row
+// mode of the layout (paged with a power-of-2 page, paged with any page,
+// contiguous). fresh: the appending decode's form (NEW; half storage only).
+template <typename T, int D>
 void launch_stream(bool paged, int page_shift, int nseg, hipStream_t s, const T* q,
                    const T* k, const T* v, const int* table, const int* lens, float* ws_ml,
                    float* ws_acc, long long* pref, T* out, int batch, int hq, int hkv,
                    int group, int rows_or_page, int tbl_width, int span, float scale_log2,
-                   int min_seg, bool fresh, bool halve) {
-    auto go = [&](auto kernel, const int* tbl, int shift, int width) {
-        kernel<<<(unsigned)nseg, 256, 0, s>>>(q, k, v, tbl, lens, ws_ml, ws_acc, pref, out,
-                                              batch, hq, hkv, group, rows_or_page, shift,
-                                              width, span, scale_log2, min_seg, halve ? 1 : 0);
+                   int min_seg, int low_seg, bool fresh, int cus) {
+    constexpr bool kF32 = std::is_same<T, float>::value;
+    auto go = [&](auto mode, auto fresh_c, const int* tbl, int shift, int width) {
+        constexpr int MODE = decltype(mode)::value;
+        constexpr bool NEW = decltype(fresh_c)::value;
+        auto launch = [&](auto kernel) {
+            kernel<<<(unsigned)nseg, 256, 0, s>>>(q, k, v, tbl, lens, ws_ml, ws_acc, pref, out,
+                                                  batch, hq, hkv, group, rows_or_page, shift,
+                                                  width, span, scale_log2, min_seg, low_seg, cus);
+        };
+        if constexpr (!kF32 && D == kMfmaDim) launch(attn_decode_stream<T, MODE, NEW>);
+        else launch(attn_decode_wide<T, D, MODE, NEW>);
     };
-    if (paged && page_shift >= 0) {
-        if (fresh) go(attn_decode_stream<T, kRowsPagedPow2, true>, table, page_shift, tbl_width);
-        else go(attn_decode_stream<T, kRowsPagedPow2, false>, table, page_shift, tbl_width);
+    using Paged2 = std::integral_constant<int, kRowsPagedPow2>;
+    using PagedN = std::integral_constant<int, kRowsPagedDiv>;
+    using Contig = std::integral_constant<int, kRowsContig>;
+    if (fresh) {
+        if constexpr (kF32) {
+            inval("attention: the append form is for half storage");
+        } else {
+            if (!paged) inval("attention: the append form is paged only");
+            if (page_shift >= 0) go(Paged2{}, std::true_type{}, table, page_shift, tbl_width);
+            else go(PagedN{}, std::true_type{}, table, -1, tbl_width);
+        }
+    } else if (paged && page_shift >= 0) {
+        go(Paged2{}, std::false_type{}, table, page_shift, tbl_width);
     } else if (paged) {
-        if (fresh) go(attn_decode_stream<T, kRowsPagedDiv, true>, table, -1, tbl_width);
-        else go(attn_decode_stream<T, kRowsPagedDiv, false>, table, -1, tbl_width);
+        go(PagedN{}, std::false_type{}, table, -1, tbl_width);
     } else {
-        if (fresh) inval("attention: the append form is paged only");
-        go(attn_decode_stream<T, kRowsContig, false>, nullptr, -1, 0);
+        go(Contig{}, std::false_type{}, nullptr, -1, 0);
     }
 }
 
@@ -1085,6 +1529,10 @@ struct Workspace {
     // to the static per-device array of FT_NOALLOC_WORKSPACE_BYTES; the paged
     // decode raises instead, as the reference's (attention.cu:1830-1844)
     void* (*fallback)() = nullptr;
+    // bytes that are there whatever happens to an allocation
+    size_t sure() const {
+        return fixed ? cap : fallback ? (size_t)FT_NOALLOC_WORKSPACE_BYTES : SIZE_MAX;
+    }
     void* get(size_t bytes, hipStream_t s) const {
         if (!fixed) {
             try {
@@ -1102,11 +1550,65 @@ struct Workspace {
     }
 };
 
-template <typename T>
+// One decode call on the stream kernels (stream_eligible, span > 0).
 // Returns 0, or 1 when the combine kernel wrote the per-head maxima into
 // amax, or 2 when it also folded them and wrote the int8 codes of the
 // output into qcodes and the scale into *qscale (quantize_int8's; the
 // stream path with every combine workgroup resident at once).
+template <typename T, int D>
+int attention_stream_run(const T* q, const T* k, const T* v, const int* table, const int* lens,
+                         T* out, int batch, int hq, int hkv, int rows_or_page, int page_shift,
+                         int tbl_width, bool paged, int span, float scale_log2, int nseg,
+                         int min_seg, int low_seg, int cus, char* ws, hipStream_t s, float* amax,
+                         signed char* qcodes, float* qscale, const AppendArgs<T>& ap) {
+    const int group = hq / hkv;
+    const size_t nslots = ((size_t)nseg + (size_t)batch * hkv) * group;
+    float* ws_ml = (float*)ws;
+    float* ws_acc = ws_ml + ((nslots * 2 + 63) & ~(size_t)63);
+    long long* pref = (long long*)(ws_acc + nslots * D);
+    if (ap.k_new && (amax || qcodes)) inval("attention: the append form keeps no per-head maxima");
+    launch_stream<T, D>(paged, page_shift, nseg, s, q, k, v, table, lens, ws_ml, ws_acc, pref,
+                        out, batch, hq, hkv, group, rows_or_page, tbl_width, span, scale_log2,
+                        min_seg, low_seg, ap.k_new != nullptr, cus);
+    launch_check("attention decode kernel launch");
+    const long long heads = (long long)batch * hq;
+    if (ap.k_new) {
+        if (page_shift >= 0)
+            attn_combine_append<T, D, kRowsPagedPow2><<<(unsigned)heads, 64, 0, s>>>(
+                ws_ml, ws_acc, pref, lens, q, ap, table, out, batch, hq, hkv, group, span,
+                rows_or_page, page_shift, tbl_width, scale_log2);
+        else
+            attn_combine_append<T, D, kRowsPagedDiv><<<(unsigned)heads, 64, 0, s>>>(
+                ws_ml, ws_acc, pref, lens, q, ap, table, out, batch, hq, hkv, group, span,
+                rows_or_page, -1, tbl_width, scale_log2);
+        launch_check("attention combine + append kernel launch");
+        return 0;
+    }
+    if (qcodes) {
+        const long long nwg = (heads + kCqWaves - 1) / kCqWaves;
+        if (nwg <= (1 << 16)) {
+            const GridMax gm = gridmax_state((int)nwg, s);
+            if (grid_resident((const void*)attn_combine_quant<T, D>, (int)nwg, 64 * kCqWaves,
+                              GridUse::AttnOut)) {
+                attn_combine_quant<T, D><<<(unsigned)nwg, 64 * kCqWaves, 0, s>>>(
+                    ws_ml, ws_acc, pref, out, qcodes, qscale, batch, hq, hkv, group, gm);
+                launch_check("attention combine + quantize kernel launch");
+                return 2;
+            }
+        }
+    }
+    if (amax)
+        attn_combine_stream<T, D, true><<<(unsigned)heads, 64, 0, s>>>(
+            ws_ml, ws_acc, pref, out, amax, batch, hq, hkv, group, 0);
+    else
+        attn_combine_stream<T, D, false><<<(unsigned)heads, 64, 0, s>>>(
+            ws_ml, ws_acc, pref, out, nullptr, batch, hq, hkv, group, 0);
+    launch_check("attention combine kernel launch");
+    return amax ? 1 : 0;
+}
+
+// As attention_stream_run, whatever the shape.
+template <typename T>
 int attention_run(const T* q, const T* k, const T* v, const int* table,
                    const int* lens, T* out, int batch, int hq, int hkv,
                    int rows_or_page, int tbl_width, int dim, bool paged,
@@ -1132,8 +1634,6 @@ int attention_run(const T* q, const T* k, const T* v, const int* table,
     if (!q || !out || (span > 0 && (!k || !v)) || (paged && span > 0 && !table))
         inval("attention: null operand");
     const int group = hq / hkv;
-    const bool fast = mfma_eligible(q, k, v, group, dim) && batch <= kStreamScanRows &&
-                      tune(Tune::AttnForceGeneric, 0) == 0;
     int page_shift = -1;
     if (paged && (rows_or_page & (rows_or_page - 1)) == 0) {
         int sh = 0;
@@ -1141,82 +1641,55 @@ int attention_run(const T* q, const T* k, const T* v, const int* table,
         page_shift = sh;
     }
     const float scale_log2 = (1.0f / sqrtf((float)dim)) * kLog2e;
-    if constexpr (!std::is_same<T, float>::value) {
-        if (fast && span > 0) {
-            // stream split: G equal token segments, G = 2 workgroups per CU
-            // (the kernel's register budget allows exactly two per CU); the
-            // kernel takes one per CU for long rows of equal length unless
-            // FT_ATTN_SEGS sets the count
-            const int forced = tune(Tune::AttnSegs, 0);
-            int nseg = forced > 0 ? forced : 2 * dev_info().cu_count;
-            nseg = std::max(1, std::min(nseg, 1 << 20));
-            const bool halve = forced <= 0;
-            const int min_seg = std::max(32, tune(Tune::AttnMinSeg, kStreamMinSeg));
-            const size_t nslots = ((size_t)nseg + (size_t)batch * hkv) * group;
-            const size_t ml_floats = (nslots * 2 + 63) & ~(size_t)63;
-            const size_t acc_floats = nslots * dim;
-            char* ws = (char*)wsp.get(
-                (ml_floats + acc_floats) * sizeof(float) + (batch + 2) * sizeof(long long), s);
-            float* ws_ml = (float*)ws;
-            float* ws_acc = ws_ml + ml_floats;
-            long long* pref = (long long*)(ws_acc + acc_floats);
-            if (ap.k_new && (amax || qcodes))
-                inval("attention: the append form keeps no per-head maxima");
-            launch_stream<T>(paged, page_shift, nseg, s, q, k, v, table, lens, ws_ml, ws_acc,
-                             pref, out, batch, hq, hkv, group, rows_or_page, tbl_width,
-                             (int)span, scale_log2, min_seg, ap.k_new != nullptr, halve);
-            launch_check("attention decode kernel launch");
-            if (ap.k_new) {
-                const unsigned grid = (unsigned)((long long)batch * hq);
-                if (page_shift >= 0)
-                    attn_combine_append<T, kRowsPagedPow2><<<grid, 64, 0, s>>>(
-                        ws_ml, ws_acc, pref, lens, q, ap, table, out, batch, hq, hkv, group,
-                        min_seg, (int)span, rows_or_page, page_shift, tbl_width, scale_log2);
-                else
-                    attn_combine_append<T, kRowsPagedDiv><<<grid, 64, 0, s>>>(
-                        ws_ml, ws_acc, pref, lens, q, ap, table, out, batch, hq, hkv, group,
-                        min_seg, (int)span, rows_or_page, -1, tbl_width, scale_log2);
-                launch_check("attention combine + append kernel launch");
-                return 0;
-            }
-            if (qcodes) {
-                const long long heads = (long long)batch * hq;
-                const long long nwg = (heads + kCqWaves - 1) / kCqWaves;
-                if (nwg <= (1 << 16)) {
-                    const GridMax gm = gridmax_state((int)nwg, s);
-                    if (grid_resident((const void*)attn_combine_quant<T>, (int)nwg,
-                                      64 * kCqWaves, GridUse::AttnOut)) {
-                        attn_combine_quant<T><<<(unsigned)nwg, 64 * kCqWaves, 0, s>>>(
-                            ws_ml, ws_acc, pref, out, qcodes, qscale, batch, hq, hkv, group,
-                            min_seg, gm);
-                        launch_check("attention combine + quantize kernel launch");
-                        return 2;
-                    }
-                }
-            }
-            if (amax)
-                attn_combine_stream<T, true><<<(unsigned)((long long)batch * hq), 64, 0, s>>>(
-                    ws_ml, ws_acc, pref, out, amax, batch, hq, hkv, group, min_seg, 0);
-            else
-                attn_combine_stream<T, false><<<(unsigned)((long long)batch * hq), 64, 0, s>>>(
-                    ws_ml, ws_acc, pref, out, nullptr, batch, hq, hkv, group, min_seg, 0);
-            launch_check("attention combine kernel launch");
-            return amax ? 1 : 0;
+    // the general kernel's split (also what the stream kernels' workspace is
+    // held against when only a bounded one is at hand)
+    const long long target = (long long)dev_info().cu_count * 16;
+    int chunk = choose_chunk(batch, hkv, span, 64, kGenMaxChunk, target);
+    const int forced_chunk = tune(Tune::AttnChunk, 0);
+    if (forced_chunk > 0) chunk = std::min(forced_chunk, kGenMaxChunk);
+    const int cmax = span > 0 ? (int)((span + chunk - 1) / chunk) : 1;
+    const long long units = (long long)batch * hkv * cmax;
+    auto ws_bytes = [&](size_t nslots) {
+        return (((nslots * 2 + 63) & ~(size_t)63) + nslots * dim) * sizeof(float);
+    };
+    const size_t gen_bytes = ws_bytes((size_t)units * group);
+
+    if (stream_eligible(q, k, v, group, dim) && batch <= kStreamScanRows && span > 0 &&
+        tune(Tune::AttnForceGeneric, 0) == 0) {
+        // stream split: G equal token segments, G = 2 workgroups per CU
+        // (the kernel's register budget allows exactly two per CU); the
+        // kernel takes one per CU for long rows of equal length unless
+        // FT_ATTN_SEGS sets the count
+        const int forced = tune(Tune::AttnSegs, 0);
+        const int cu_count = dev_info().cu_count;
+        const bool one_per_cu = std::is_same<T, float>::value && dim == kMfmaDim;  // kOccupancy
+        int nseg = forced > 0 ? forced : one_per_cu ? cu_count : 2 * cu_count;
+        nseg = std::max(1, std::min(nseg, 1 << 20));
+        const int cus = forced > 0 ? 0 : cu_count;
+        const int tuned_seg = tune(Tune::AttnMinSeg, 0);
+        const int min_seg = std::max(32, tuned_seg > 0 ? tuned_seg : kStreamMinSeg);
+        const int low_seg = tuned_seg > 0 ? min_seg : kStreamLowSeg;
+        const size_t bytes = ws_bytes(((size_t)nseg + (size_t)batch * hkv) * group) +
+                             (batch + 2) * sizeof(long long);
+        // a bounded workspace that only the general kernel's partials fit
+        const bool half128 = !std::is_same<T, float>::value && dim == kMfmaDim;
+        if (half128 || bytes <= wsp.sure() || gen_bytes > wsp.sure()) {
+            char* ws = (char*)wsp.get(bytes, s);
+            if (dim == kMfmaDim)
+                return attention_stream_run<T, 128>(
+                    q, k, v, table, lens, out, batch, hq, hkv, rows_or_page, page_shift,
+                    tbl_width, paged, (int)span, scale_log2, nseg, min_seg, low_seg, cus, ws, s,
+                    amax, qcodes, qscale, ap);
+            return attention_stream_run<T, 64>(
+                q, k, v, table, lens, out, batch, hq, hkv, rows_or_page, page_shift, tbl_width,
+                paged, (int)span, scale_log2, nseg, min_seg, low_seg, cus, ws, s, amax, qcodes,
+                qscale, ap);
         }
     }
     if (ap.k_new) inval("attention: the append form runs on the stream kernel only");
-    const long long target = (long long)dev_info().cu_count * 16;
-    int chunk = choose_chunk(batch, hkv, span, 64, kGenMaxChunk, target);
-    const int forced = tune(Tune::AttnChunk, 0);
-    if (forced > 0) chunk = std::min(forced, kGenMaxChunk);
-    const int cmax = span > 0 ? (int)((span + chunk - 1) / chunk) : 1;
-    const long long units = (long long)batch * hkv * cmax;
     if (units * 256 > (1LL << 31)) inval("attention problem too large for one launch");
-    const size_t nslots = (size_t)units * group;
-    const size_t ml_floats = (nslots * 2 + 63) & ~(size_t)63;
-    float* ws = (float*)wsp.get((ml_floats + nslots * dim) * sizeof(float), s);
-    float* ws_ml = ws;
-    float* ws_acc = ws + ml_floats;
+    float* ws_ml = (float*)wsp.get(gen_bytes, s);
+    float* ws_acc = ws_ml + (((size_t)units * group * 2 + 63) & ~(size_t)63);
     RowMap rm;
     rm.table = paged ? table : nullptr;
     rm.hkv = hkv;
@@ -1314,7 +1787,7 @@ __global__ __launch_bounds__(256) void lens_plus1_kernel(const int* __restrict__
 
 // kv_append_paged(k_pool, v_pool, table, k_new, v_new, lens) followed by
 // attention_decode_paged(q, k_pool, v_pool, table, lens + 1), in one call.
-// On the stream path (bf16 / fp16, D = 128) the decode
+// On the stream path (bf16 / fp16, D = 64 or 128) the decode
 // kernel attends the lens[b] cached tokens (every piece leaves a partial)
 // and attn_combine_append folds the fresh token from k_new / v_new into
 // each row's log-sum-exp merge (float32) and writes it to the pools - one
@@ -1329,7 +1802,7 @@ void attention_append_run(const T* q, T* k_pool, T* v_pool, const int* table, co
     const long long span = (long long)tbl_width * page;
     const int group = hkv > 0 ? hq / hkv : 0;
     const bool fast = !std::is_same<T, float>::value && hkv > 0 && hq % hkv == 0 &&
-                      mfma_eligible(q, k_pool, v_pool, group, dim) &&
+                      stream_eligible(q, k_pool, v_pool, group, dim) &&
                       (uintptr_t)k_new % 16 == 0 && (uintptr_t)v_new % 16 == 0 &&
                       batch <= kStreamScanRows && tune(Tune::AttnForceGeneric, 0) == 0 &&
                       span > 0 && page >= 1 && tbl_width >= 0;

@@ -134,19 +134,6 @@ __device__ __forceinline__ bool f16_tile_ok(us2_t mx) {
     return !too_big && has_scale;
 }
 
-// maximum over lanes l, l ^ 16, l ^ 32, l ^ 48 without LDS: with both
-// operands x, v_permlane32_swap leaves x[l] and x[l ^ 32] in the two
-// results of every lane (lanes < 32: (x[l], x[l + 32]); lanes >= 32:
-// (x[l - 32], x[l])), v_permlane16_swap likewise x[l] and x[l ^ 16]
-__device__ __forceinline__ float max4_rows(float x) {
-    const unsigned u = __float_as_uint(x);
-    const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const unsigned w = __float_as_uint(y);
-    const auto c = __builtin_amdgcn_permlane16_swap(w, w, false, false);
-    return fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
-}
-
 // V of bf16 inputs converted to fp16 once per call (one workgroup per
 // 64-key tile of a (b, kv head) slab), with a flag per tile: 1 when the
 // tile's largest |v| is in [2^-8, 2^16) (f16_tile_ok: the tile then takes

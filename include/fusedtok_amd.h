@@ -158,7 +158,7 @@ int ft_attention_decode_paged_launch_bf16_noalloc(const void* q, const void* k_p
  * out, ...) in one call (reference: the two ops, attention.cu:1924-1966
  * then 1785-1900; lens is not modified). dtype FT_DT_F32 / BF16 / F16 for
  * q, the pools, k_new / v_new [batch, kv_heads, dim] and out. For bf16 /
- * fp16 with dim 128 the decode kernel attends the lens[b] cached
+ * fp16 with dim 64 or 128 the decode kernel attends the lens[b] cached
  * tokens, and its combine kernel folds the fresh token's
  * score and value into each row's log-sum-exp merge (in float32, so out
  * equals the two ops' within the attention tolerance, not bit for bit)

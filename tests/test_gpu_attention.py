@@ -563,3 +563,113 @@ def test_paged_staged_host_inputs():
     np.testing.assert_allclose(out, oracle.attention_decode_paged(q, kp, vp, tbl, ln),
                                rtol=1e-4, atol=1e-5)
     np.testing.assert_allclose(out[0, 0], vp[tbl[0, 0], 0, 0], atol=1e-6)
+
+
+# ---------------------------------------------------------------------------
+# attn_decode_wide: half storage with D = 64, float32 with D = 64 and 128
+# ---------------------------------------------------------------------------
+WIDE = [(torch.bfloat16, 64), (torch.float16, 64), (torch.float32, 64), (torch.float32, 128)]
+
+
+def assert_wide_close(got, ref, dt, what):
+    if dt is torch.float32:  # the float32 bar of this file
+        np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-5, err_msg=what)
+    else:
+        assert_half_close(got, ref, what)
+
+
+@pytest.mark.parametrize("dt,d", WIDE)
+@pytest.mark.parametrize("group", [1, 3, 4, 16])
+@pytest.mark.parametrize("page", [0, 5, 16])
+def test_wide_decode_matches_oracle(dt, d, group, page, tuning):
+    # lengths around the 16- and 32-token steps, the 4 waves' round (64 /
+    # 128) and the segments (32, the default and what a small call takes);
+    # page 0: contiguous. The rows past each length hold NaN. A call off
+    # 16-byte alignment and one on the general kernel agree with it.
+    if page and group == 3:
+        pytest.skip("paged decode takes group sizes 1/2/4/8/16")
+    lens = [0, 1, 15, 16, 17, 31, 32, 33, 63, 65, 127, 129, 700]
+    rng = np.random.default_rng(group * 100 + page + d)
+    b, hkv = len(lens), 2
+    ln = np.array(lens, np.int32)
+    if page:
+        q, kp, vp, tbl, _ = paged_case(rng, b, hkv * group, hkv, d, [705] * b, page=page)
+        ref = oracle.attention_decode_paged(rounded(q, dt), rounded(kp, dt), rounded(vp, dt),
+                                            tbl, ln)
+        for i, n in enumerate(lens):
+            for tok in range(n, tbl.shape[1] * page):
+                kp[tbl[i, tok // page], :, tok % page] = np.nan
+                vp[tbl[i, tok // page], :, tok % page] = np.nan
+        args = (t(kp, dt), t(vp, dt), t(tbl), t(ln))
+        call = ft.attention_decode_paged
+    else:
+        q, k, v, _ = make_case(rng, b, hkv * group, hkv, 705, d, False)
+        ref = oracle.attention_decode(rounded(q, dt), rounded(k, dt), rounded(v, dt), ln)
+        for i, n in enumerate(lens):
+            k[i, :, n:] = np.nan
+            v[i, :, n:] = np.nan
+        args = (t(k, dt), t(v, dt), t(ln))
+        call = ft.attention_decode
+    qt = t(q, dt)
+    shifted = torch.empty(qt.numel() + 1, dtype=dt, device=DEV)[1:].view_as(qt).copy_(qt)
+    for what, qq, switch in (("default", qt, None), ("segments of 32", qt, ("FT_ATTN_MIN_SEG", 32)),
+                             ("shifted", shifted, None),
+                             ("general", qt, ("FT_ATTN_FORCE_GENERIC", 1))):
+        if switch:
+            tuning(*switch)
+        got = call(qq, *args).float().cpu().numpy()
+        if switch:
+            tuning.clear(switch[0])
+        assert (got[0] == 0).all()
+        assert_wide_close(got, ref, dt, what)
+
+
+@pytest.mark.parametrize("dt,d", WIDE)
+def test_wide_decode_values_that_are_not_finite_stay_in_their_column(dt, d, tuning):
+    # an infinite V value reaches its own output column alone, at the end of
+    # a piece and inside one, as on the general kernel; a NaN key makes its
+    # row NaN
+    rng = np.random.default_rng(d)
+    q, k, v, _ = make_case(rng, 3, 8, 2, 200, d, False)
+    lens = np.array([77, 200, 130], np.int32)
+    v[0, :, 76, 5] = np.inf
+    v[1, :, 40, 9] = -np.inf
+    k[2, 1, 129] = np.nan
+    args = (t(q, dt), t(k, dt), t(v, dt), t(lens))
+    got = ft.attention_decode(*args).float().cpu().numpy()
+    tuning("FT_ATTN_FORCE_GENERIC", 1)
+    ref = ft.attention_decode(*args).float().cpu().numpy()
+    assert np.isposinf(got[0, :, 5]).all() and np.isneginf(got[1, :, 9]).all()
+    assert np.isnan(got[2, 4:]).all() and np.isfinite(got[2, :4]).all()
+    np.testing.assert_allclose(got, ref, rtol=1e-2, atol=2e-3)
+
+
+@pytest.mark.parametrize("dt", HALF)
+def test_append_decode_of_64_dims(dt):
+    # the appending form at D = 64: pools bit for bit, the output at the
+    # attention bar, an empty row exactly the fresh V; replayed from a graph
+    rng = np.random.default_rng(64)
+    lens = np.array([0, 1, 16, 40, 333, 1027], np.int32)
+    b, hkv, group, d = len(lens), 2, 4, 64
+    q, kp, vp, tbl, _ = paged_case(rng, b, hkv * group, hkv, d, [1040] * b, page=16)
+    kn = rng.standard_normal((b, hkv, d)).astype(np.float32)
+    vn = rng.standard_normal((b, hkv, d)).astype(np.float32)
+    k1, v1 = t(kp, dt), t(vp, dt)
+    k2, v2 = k1.clone(), v1.clone()
+    args = (t(q, dt), k1, v1, t(tbl), t(kn, dt), t(vn, dt), t(lens))
+    out = ft.attention_decode_paged_append(*args)
+    ft.kv_append_paged(k2, v2, args[3], args[4], args[5], args[6])
+    assert torch.equal(k1, k2) and torch.equal(v1, v2)
+    ref = oracle.attention_decode_paged(rounded(q, dt), k2.float().cpu().numpy(),
+                                        v2.float().cpu().numpy(), tbl, lens + 1)
+    assert_half_close(out.float().cpu().numpy(), ref)
+    assert torch.equal(out[0].view(hkv, group, d), args[5][0].unsqueeze(1).expand(hkv, group, d))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        again = ft.attention_decode_paged_append(*args)
+    for _ in range(3):
+        again.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(again, out)
+        ft.attention_decode_paged(args[0], k1, v1, args[3], args[6])  # eager work between
