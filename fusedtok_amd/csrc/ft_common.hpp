@@ -117,6 +117,8 @@ enum class Tune : int {
                            // to fold inside one launch (grid_max), which then
                            // take their two-launch forms: 1 all, 2 SwiGLU,
                            // 4 attention output, 8 RMSNorm
+    QgemmMid,              // FT_QGEMM_MID: mid-size GEMM kernel: -1 off, else
+                           // 100 ksplit + 10 MI + NJ (qgemm_mid's tile)
     kCount
 };
 // The switch's value, or `dflt` when it is neither in the environment nor

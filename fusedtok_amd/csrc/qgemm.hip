@@ -34,8 +34,12 @@
 //                  v_mfma_i32_32x32x32_i8 fed by a 5-stage global->LDS DMA
 //                  ring; LDS-staged, coalesced epilogue.
 //   qgemm_big      M, N >= 256, other K: the same tiles, register-staged.
-//   qgemm_tiled    64 < M (< 256 or N < 256): 128x128 tiles, 64-byte slabs
-//                  double-buffered through LDS.
+//   qgemm_mid      64 < M, K % 64 == 0, where its estimate beats the 256x256
+//                  tiles' (mid_pick, big_us): 128-256 row x 64 / 128 column
+//                  tiles, K split to fill the CUs, 128-byte K slabs DMA'd
+//                  global->LDS into a 3- or 4-slab ring.
+//   qgemm_tiled    64 < M (< 256 or N < 256), other K: 128x128 tiles, 64-byte
+//                  slabs double-buffered through LDS.
 //   qgemm_scalar   any shape/alignment (K % 16 != 0, misaligned views).
 //   K == 0         zero fill (a kernel, not a memset, so it captures cleanly).
 #include "ft_common.hpp"
@@ -79,6 +83,14 @@ __device__ __forceinline__ i32x4 lds_read16(unsigned addr) {
     return v;
 }
 
+// Blocks go round the 8 XCDs: block t of `total` -> its place in an order in
+// which each XCD's blocks are consecutive (XCD t % 8 takes the run number
+// t % 8, the first total % 8 runs one longer).
+__device__ __forceinline__ int xcd_order(int t, int total) {
+    const int x = t & 7;
+    return x * (total >> 3) + min(x, total & 7) + (t >> 3);
+}
+
 struct Epi {
     void* y;
     float sa;
@@ -109,6 +121,37 @@ __device__ __forceinline__ void epi_store_scaled(const Epi& e, int n, int row, i
         if constexpr (OUT == kOutF32) static_cast<float*>(e.y)[idx] = val;
         if constexpr (OUT == kOutBF16) static_cast<bf16*>(e.y)[idx] = (bf16)val;
         if constexpr (OUT == kOutF16) static_cast<f16*>(e.y)[idx] = (f16)val;
+    }
+}
+
+// epi_store_scaled of 4 consecutive columns from col on (scales sc): one 8-
+// or 16-byte store where rows are a multiple of 4 columns
+template <int OUT>
+__device__ __forceinline__ void store4(const Epi& e, int n, int row, int col, i32x4 acc,
+                                       const float (&sc)[4]) {
+    if (n % 4 != 0) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (col + c < n) epi_store_scaled<OUT>(e, n, row, col + c, acc[c], sc[c]);
+        return;
+    }
+    const size_t idx = (size_t)row * n + col;
+    if constexpr (OUT == kOutI32) {
+        *reinterpret_cast<i32x4*>(static_cast<int*>(e.y) + idx) = acc;
+    } else {
+        float v[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            v[c] = (float)acc[c] * sc[c];
+            asm("" : "+v"(v[c]));
+        }
+        if constexpr (OUT == kOutF32) {
+            *reinterpret_cast<float4*>(static_cast<float*>(e.y) + idx) =
+                make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+            using T = std::conditional_t<OUT == kOutBF16, bf16, f16>;
+            St<T>::st4(static_cast<T*>(e.y) + idx, make_float4(v[0], v[1], v[2], v[3]));
+        }
     }
 }
 
@@ -1771,8 +1814,7 @@ void qgemm_big_w16(const i8* __restrict__ a, const i8* __restrict__ b, Epi e,
     // of 8), and the tiles one XCD holds at once form a block of `band` tile
     // rows, so they share A and B panels in that XCD's L2
     auto tile_origin = [&](int t, int& bm, int& bn) {
-        int pid = t;
-        if (ntiles % 8 == 0) pid = (pid % 8) * (ntiles / 8) + pid / 8;
+        const int pid = xcd_order(t, ntiles);
         const int bi = pid / (band * tn);
         const int first_m = bi * band;
         const int band_m = min(tm - first_m, band);
@@ -1954,6 +1996,223 @@ void qgemm_big_w16(const i8* __restrict__ a, const i8* __restrict__ b, Epi e,
 }
 
 // ---------------------------------------------------------------------------
+// mid (more rows than the skinny kernel takes, too few tiles for the
+// 256 x 256 one): BM x BN tiles, BM = 64 MI rows (128, 192 or 256) by
+// BN = 32 NJ columns (64 or 128), one workgroup of 8 waves per tile and K
+// split, two waves per SIMD. Wave (wm, wn) of 4 x 2 owns MI x NJ blocks of
+// v_mfma_i32_16x16x64_i8 (C^T: a lane holds 4 consecutive columns of a row,
+// as in qgemm_big_w16).
+//
+// What bounds it: with one tile of rows the weights are read once (HBM, 12
+// us for 14336 x 4096 at 5 TB/s); beyond, the operand traffic L2 -> LDS (about
+// 30 B per clock and CU), which BM rows a tile keeps at (BM + BN) * 128 bytes
+// per BM * BN * 128 MACs. 128-byte K slabs arrive by global -> LDS DMA in
+// whole lines (8 rows an instruction) through a ring of NST slabs, NST - 1
+// in flight - the tiled kernel before it held one 64-byte slab in registers.
+// LDS rows are 128 bytes, chunk c of row r at c ^ ((r >> 1) & 7): conflict-
+// free fragment reads. One barrier per slab. K % 128 = 64 leaves a half slab
+// at the end, whose second half is neither read past the row nor multiplied.
+//
+// Rows past M / N read a clamped (real) row, whose products are not stored.
+// The tiles that share weight columns are consecutive on one XCD. ksplit > 1:
+// int32 partials [ks][m][n] for qgemm_ksum4.
+//
+// Measured (graph replays, weights cycled past the last-level cache, best
+// tile, us before -> now): N 14336, K 4096: M 65 55 -> 18, 150 57 -> 23, 300
+// 48 -> 32, 512 54 -> 38; N 4096, K 4096: M 150 52 -> 14, 1000 50 -> 26; N
+// 4096, K 14336: M 150 158 -> 25, 1000 161 -> 71 (before: qgemm_tiled below
+// 256 rows, 256 x 256 tiles on a quarter of the CUs or fewer from there).
+// ---------------------------------------------------------------------------
+template <int MI, int NJ>
+struct MidCfg {
+    static constexpr int kBM = 64 * MI, kBN = 32 * NJ;
+    static constexpr int kSlab = (kBM + kBN) * kK2;              // bytes
+    static constexpr int kIns = (kBM + kBN) / 8 / 8;             // DMA per wave and slab
+    static constexpr int kFit = (160 << 10) / kSlab;
+    static constexpr int kStages = kFit > 4 ? 4 : kFit;
+    static_assert((kBM + kBN) % 64 == 0 && kStages >= 3, "tile");
+};
+
+template <int N>
+__device__ __forceinline__ void wait_lgkm() {
+    static_assert(N >= 0 && N < 16, "lgkmcnt range");
+    asm volatile("s_waitcnt lgkmcnt(%0)" : : "n"(N) : "memory");
+}
+
+// one slab's DMA by one wave: its IN instructions, 64 rows of LDS apart
+template <int IN>
+__device__ __forceinline__ void mid_issue(const i8* const (&src)[IN], int off, i8* dst) {
+#pragma unroll
+    for (int i = 0; i < IN; ++i) {
+        const i8* from = src[i] + off;
+        __builtin_amdgcn_global_load_lds(from, (lds_void_p)(dst + 64 * i * kK2), 16, 0, 0);
+    }
+}
+
+template <int MI, int NJ, int OUT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void qgemm_mid(const i8* __restrict__ a, const i8* __restrict__ b, Epi e, int m, int n, int k,
+               int tm, int tiles, int ksplit, int* __restrict__ part) {
+    using C = MidCfg<MI, NJ>;
+    constexpr int BM = C::kBM, BN = C::kBN, NST = C::kStages, kIns = C::kIns;
+    __shared__ __attribute__((aligned(16))) i8 lds[NST * C::kSlab];
+
+    // workgroup -> (K split, tile): blocks go round the 8 XCDs, each XCD
+    // takes a run of tiles, row tiles first
+    const int pid = xcd_order((int)blockIdx.x, tiles * ksplit);
+    const int ks = pid / tiles, tile = pid - ks * tiles;
+    const int bn = tile / tm * BN, bm = (tile % tm) * BM;
+    const int slabs = (k + kK2 - 1) / kK2;
+    const int per = (slabs + ksplit - 1) / ksplit;
+    const int s0 = min(slabs, ks * per), s1 = min(slabs, s0 + per);
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int r16 = lane & 15, q4 = lane >> 4;
+
+    // DMA instruction i of this wave fills slab rows 8 (wave + 8 i) .. + 7 (A's
+    // BM rows, then B's BN); lane l brings chunk (l & 7) ^ swz of row l >> 3
+    const int ch = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
+    const i8* src[kIns];
+#pragma unroll
+    for (int i = 0; i < kIns; ++i) {
+        const int row = 8 * (wave + 8 * i) + (lane >> 3);
+        src[i] = 8 * (wave + 8 * i) < BM ? a + (size_t)min(bm + row, m - 1) * k
+                                         : b + (size_t)min(bn + row - BM, n - 1) * k;
+    }
+    auto issue = [&](int kt, int st) {
+        // the half slab at the end of K: its missing chunks repeat a real one
+        mid_issue<kIns>(src, min(kt * kK2 + 16 * ch, k - 16),
+                        lds + st * C::kSlab + 8 * wave * kK2);
+    };
+
+    i32x4 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
+
+    const unsigned lds0 = lds_addr(lds);
+    unsigned fa0[2], fb0[2];  // fragment bases of the two 64-byte sub-steps
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const unsigned sw = 16u * ((4 * u + q4) ^ ((r16 >> 1) & 7));
+        fa0[u] = lds0 + (unsigned)((16 * MI * wm + r16) * kK2) + sw;
+        fb0[u] = lds0 + (unsigned)((BM + 16 * NJ * wn + r16) * kK2) + sw;
+    }
+
+#pragma unroll
+    for (int j = 0; j < NST - 1; ++j)
+        if (s0 + j < s1) issue(s0 + j, j);
+    int st = 0;
+    for (int kt = s0; kt < s1; ++kt) {
+        // this wave's copies of slab kt have landed (later ones may fly) ...
+        if (kt + NST - 2 < s1) wait_vmcnt<(NST - 2) * kIns>();
+        else if (NST > 3 && kt + 1 < s1) wait_vmcnt<kIns>();
+        else wait_vmcnt<0>();
+        // ... and after the barrier everyone's; slab kt - 1's stage is free
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + NST - 1 < s1) issue(kt + NST - 1, st == 0 ? NST - 1 : st - 1);
+        const unsigned base = (unsigned)(st * C::kSlab);
+        i32x4 fa[2][MI], fb[2][NJ];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) fb[u][j] = lds_read16(fb0[u] + base + 16 * kK2 * j);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) fa[u][i] = lds_read16(fa0[u] + base + 16 * kK2 * i);
+        }
+        const bool half = kt * kK2 + kK2 > k;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            // sub-step u's fragments (LDS reads return in order)
+            __builtin_amdgcn_sched_barrier(0);
+            if (u == 0) wait_lgkm<MI + NJ>();
+            else wait_lgkm<0>();
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(fb[u][j]));
+#pragma unroll
+            for (int i = 0; i < MI; ++i) asm volatile("" : "+v"(fa[u][i]));
+            __builtin_amdgcn_sched_barrier(0);
+            if (u == 1 && half) break;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[u][j], fa[u][i],
+                                                                      acc[i][j], 0, 0, 0);
+        }
+        st = st + 1 == NST ? 0 : st + 1;
+    }
+
+    const float sa = ksplit == 1 ? epi_sa(e) : 0.0f;
+    int* const mine = ksplit == 1 ? nullptr : part + (size_t)ks * m * n;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int col = bn + 16 * (NJ * wn + j) + 4 * q4;
+        if (col >= n) continue;
+        float sc[4] = {0.f, 0.f, 0.f, 0.f};
+        if (OUT != kOutI32 && ksplit == 1) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                sc[c] = e.sb_vec ? sa * e.sb_vec[min(col + c, n - 1)] : sa * e.sb;
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const int row = bm + 16 * (MI * wm + i) + r16;
+            if (row >= m) continue;
+            if (ksplit > 1) {
+                int* dst = mine + (size_t)row * n + col;
+                if (n % 4 == 0) {
+                    *reinterpret_cast<i32x4*>(dst) = acc[i][j];
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (col + c < n) dst[c] = acc[i][j][c];
+                }
+            } else {
+                store4<OUT>(e, n, row, col, acc[i][j], sc);
+            }
+        }
+    }
+}
+
+// out[row][col .. + 3] = the fold of qgemm_ksum, 4 columns a thread (n % 4
+// == 0, 32-bit indices): no division per value and 16-byte loads, all of a
+// batch of partials issued together.
+template <int OUT>
+__global__ __launch_bounds__(256) void qgemm_ksum4(const int* __restrict__ part, Epi e, int m,
+                                                   int n, int ksplit) {
+    const unsigned idx = blockIdx.x * 256 + threadIdx.x;
+    const unsigned n4 = (unsigned)n >> 2;
+    if (idx >= (unsigned)m * n4) return;
+    const int row = (int)(idx / n4), col = (int)(idx - row * n4) * 4;
+    const float sa = OUT == kOutI32 ? 0.0f : epi_sa(e);
+    float sc[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (OUT != kOutI32) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sc[c] = e.sb_vec ? sa * e.sb_vec[col + c] : sa * e.sb;
+    }
+    const size_t mn4 = (size_t)m * n4;
+    const i32x4* p = reinterpret_cast<const i32x4*>(part) + idx;
+    i32x4 sum = {0, 0, 0, 0};
+    for (int j0 = 0; j0 < ksplit; j0 += kKsumBatch) {
+        i32x4 v[kKsumBatch];
+#pragma unroll
+        for (int u = 0; u < kKsumBatch; ++u) {
+            const i32x4 z = {0, 0, 0, 0};
+            v[u] = j0 + u < ksplit ? p[(size_t)(j0 + u) * mn4] : z;
+        }
+#pragma unroll
+        for (int u = 0; u < kKsumBatch; ++u) sum += v[u];
+    }
+    store4<OUT>(e, n, row, col, sum, sc);
+}
+
+// ---------------------------------------------------------------------------
 // dispatch
 // ---------------------------------------------------------------------------
 // reference qgemm.cu:599-604 bounds m*n*k <= 2^38; this build instead bounds
@@ -1966,6 +2225,117 @@ void qgemm_check(int m, int n, int k) {
 
 size_t out_elem_bytes(int out) {
     return out == kOutBF16 || out == kOutF16 ? 2 : 4;
+}
+
+// ---- qgemm_mid's tiles and K split -----------------------------------------
+// Estimated microseconds, from graph replays with the weights cycled past the
+// last-level cache (M 65-2048; N x K 14336 x 4096, 4096 x 4096, 4096 x 14336,
+// 28672 x 4096, 1584 x 2432). Over 105 random shapes (M 65-4096, N 1024-
+// 28672, K 512-14336) the pick is within 10% of the best of all tiles, splits
+// and the kernels before in all but 10 (the worst: 1.35x, a 256 x 256 pick),
+// and never more than 1% behind the kernel that ran the shape before. A launch and
+// its first and last slab cost ~3.5 us; a slab costs a workgroup kMidSlabUs
+// (operand traffic, so it goes with BM + BN); a second round of workgroups
+// runs 10% longer than two first ones. A K split adds the fold launch: 3.8
+// us and the partials written and read, from cache, at ~12 TB/s.
+struct MidPick {
+    int mi = 0, nj = 0, ksplit = 1;
+    float us = 1e30f;
+};
+constexpr float kMidSlabUs[3][2] = {{0.42f, 0.66f}, {0.55f, 0.84f}, {0.70f, 1.04f}};
+constexpr int kMidMaxSplit = 8;
+
+MidPick mid_pick(int m, int n, int k, int cus, bool may_split) {
+    MidPick best;
+    const int slabs = (k + kK2 - 1) / kK2;
+    for (int mi = 2; mi <= 4; ++mi) {
+        for (int nj = 2; nj <= 4; nj += 2) {
+            const long long tiles = (long long)((m + 64 * mi - 1) / (64 * mi)) *
+                                    ((n + 32 * nj - 1) / (32 * nj));
+            for (int ks = 1; ks <= kMidMaxSplit && ks <= slabs; ++ks) {
+                if (ks > 1 && (!may_split || tiles * ks > cus)) break;
+                const long long rounds = (tiles * ks + cus - 1) / cus;
+                float us = 3.5f + (rounds > 1 ? 1.1f : 1.0f) * rounds *
+                                      ((slabs + ks - 1) / ks) * kMidSlabUs[mi - 2][nj / 2 - 1];
+                if (ks > 1) us += 3.8f + 8e-6f / 12.0f * ks * (float)m * (float)n;
+                if (us < best.us) best = MidPick{mi, nj, ks, us};
+            }
+        }
+    }
+    return best;
+}
+
+// The 256 x 256 kernel's estimate: a slab and round cost 1.25 us with few
+// tiles a round and 1.7 us with one on every CU (both operands from L2).
+float big_us(int m, int n, int k, int cus) {
+    const long long tiles = (long long)((m + kBigT - 1) / kBigT) * ((n + kBigT - 1) / kBigT);
+    const long long rounds = (tiles + cus - 1) / cus;
+    const float fill = (float)tiles / (float)(rounds * cus);
+    return 5.0f + rounds * ((k + kK2 - 1) / kK2) * (1.25f + 0.45f * fill);
+}
+
+// qgemm_mid where it is the faster kernel (more rows than the skinny kernel
+// takes; K % 64 = 0); false: nothing launched. FT_QGEMM_MID (tests): -1 off,
+// else 100 ksplit + 10 MI + NJ.
+template <int OUT>
+bool qgemm_mid_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, int k,
+                        hipStream_t s) {
+    if (k % 64 != 0 || (uintptr_t)e.y % 16 != 0 || (long long)m * n > (1LL << 31) - 1)
+        return false;
+    const int forced = tune(Tune::QgemmMid, 0);
+    const int cus = dev_info().cu_count;
+    const bool big = m >= kBigT && n >= kBigT;
+    // a test of the large kernels sets these on shapes they need not win
+    if (forced < 0 || (forced == 0 && big && (tune(Tune::QgemmBig, 0) || tune(Tune::QgemmBand, 0))))
+        return false;
+    MidPick pick;
+    if (forced > 0) {
+        pick = MidPick{forced / 10 % 10, forced % 10, std::max(1, forced / 100), 0.0f};
+        if (pick.mi < 2 || pick.mi > 4 || (pick.nj != 2 && pick.nj != 4))
+            inval("FT_QGEMM_MID: 100 ksplit + 10 MI (2..4) + NJ (2 or 4)");
+    } else {
+        pick = mid_pick(m, n, k, cus, n % 4 == 0);
+    }
+    if (forced == 0 && big && big_us(m, n, k, cus) <= pick.us) return false;
+    int* part = nullptr;
+    if (pick.ksplit > 1) {
+        try {
+            part = (int*)scratch(Scratch::GemmPartials,
+                                 (size_t)pick.ksplit * m * n * sizeof(int), s);
+        } catch (const Error& err) {
+            // no room for partials (or a capture before the first call): unsplit
+            if (err.code != FT_EHIP || forced > 0) throw;
+            pick = mid_pick(m, n, k, cus, false);
+            if (big && big_us(m, n, k, cus) <= pick.us) return false;
+        }
+    }
+    const long long tm = (m + 64 * pick.mi - 1) / (64 * pick.mi);
+    const long long tiles = tm * ((n + 32 * pick.nj - 1) / (32 * pick.nj));
+    if (tiles * pick.ksplit > (1LL << 30)) inval("qgemm problem too large for one launch");
+    const unsigned grid = (unsigned)(tiles * pick.ksplit);
+#define FT_MID(MI, NJ)                                                                       \
+    qgemm_mid<MI, NJ, OUT><<<grid, 512, 0, s>>>(a, b, e, m, n, k, (int)tm, (int)tiles,       \
+                                                pick.ksplit, part)
+    switch (10 * pick.mi + pick.nj) {
+    case 22: FT_MID(2, 2); break;
+    case 24: FT_MID(2, 4); break;
+    case 32: FT_MID(3, 2); break;
+    case 34: FT_MID(3, 4); break;
+    case 42: FT_MID(4, 2); break;
+    default: FT_MID(4, 4); break;
+    }
+#undef FT_MID
+    launch_check("qgemm mid kernel launch");
+    if (pick.ksplit > 1) {
+        if (n % 4 == 0)
+            qgemm_ksum4<OUT><<<grid_1d((long long)m * (n / 4), 256, 1 << 30), 256, 0, s>>>(
+                part, e, m, n, pick.ksplit);
+        else
+            qgemm_ksum<OUT><<<grid_1d((long long)m * n, 256, 1 << 30), 256, 0, s>>>(
+                part, e, m, n, pick.ksplit, nullptr);
+        launch_check("qgemm k-split fold launch");
+    }
+    return true;
 }
 
 template <int OUT>
@@ -2117,6 +2487,7 @@ void qgemm_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, int k,
         }
         return;
     }
+    if (force == 0 && qgemm_mid_dispatch<OUT>(a, b, e, m, n, k, s)) return;
     if ((m >= kBigT && n >= kBigT && force != 2) || force == 4) {
         const long long tiles = (long long)((m + kBigT - 1) / kBigT) * ((n + kBigT - 1) / kBigT);
         if (tiles > (1LL << 30)) inval("qgemm problem too large for one launch");

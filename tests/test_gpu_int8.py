@@ -244,6 +244,53 @@ def test_big_kernels_bit_exact(big, tuning):
     assert torch.equal(yh.cpu(), torch.from_numpy(pc).to(torch.float16))
 
 
+@pytest.mark.parametrize("tile", [22, 24, 32, 34, 42, 44])
+@pytest.mark.parametrize("ksplit", [1, 3])
+@pytest.mark.parametrize("m,n,k", [
+    (65, 63, 64),      # one half slab; rows not a multiple of 4 columns
+    (128, 64, 128),    # one whole slab, whole tiles
+    (129, 130, 192),   # a slab and a half; ragged rows and columns
+    (193, 260, 640),   # five slabs: the ring wraps, and a K split of 3 is uneven
+    (300, 132, 2112),  # many slabs, a half one last
+])
+def test_mid_kernel_bit_exact(tile, ksplit, m, n, k, tuning):
+    # every tile of the mid-size kernel (10 MI + NJ), whole and split over K,
+    # every output type, device and host activation scale
+    tuning("FT_QGEMM_MID", 100 * ksplit + tile)
+    rng = np.random.default_rng(tile * 1000 + ksplit * 100 + m)
+    a, b = rand_q(rng, m, k), rand_q(rng, n, k)
+    sb = rng.uniform(1e-3, 1e-2, n).astype(np.float32)
+    at, bt = t(a), t(b)
+    acc = ft.qgemm_i32(at, bt)
+    np.testing.assert_array_equal(acc.cpu().numpy(), oracle.qgemm_i32(a, b))
+    pc = oracle.qgemm_perchannel(a, 0.017, b, sb)
+    for odt in (torch.float32, torch.bfloat16, torch.float16):
+        y = ft.qgemm_perchannel(at, 0.017, bt, t(sb), out_dtype=odt)
+        assert torch.equal(y.cpu(), torch.from_numpy(pc).to(odt)), odt
+        y = ft.qgemm_perchannel(at, torch.tensor([0.017], device=DEV), bt, t(sb), out_dtype=odt)
+        assert torch.equal(y.cpu(), torch.from_numpy(pc).to(odt)), odt
+    np.testing.assert_array_equal(ft.qgemm(at, 0.03, bt, 0.02).cpu().numpy(),
+                                  oracle.qgemm(a, 0.03, b, 0.02))
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 4096, 4096), (150, 1024, 2432), (256, 2048, 1088),
+                                   (300, 3000, 1024), (700, 1000, 4096), (1000, 4096, 512)])
+def test_mid_choice_and_the_kernels_it_replaces_agree(m, n, k, tuning):
+    # the library's own tile and K split, the kernels these shapes ran on
+    # before, and the choice without room for partials (a capture before the
+    # first call, or an allocation that fails)
+    rng = np.random.default_rng(m + n + k)
+    at, bt = t(rand_q(rng, m, k)), t(rand_q(rng, n, k))
+    sb = t(rng.uniform(1e-3, 1e-2, n).astype(np.float32))
+    y = ft.qgemm_perchannel(at, 0.017, bt, sb, out_dtype=torch.bfloat16)
+    tuning("FT_QGEMM_MID", -1)
+    before = ft.qgemm_perchannel(at, 0.017, bt, sb, out_dtype=torch.bfloat16)
+    tuning.clear("FT_QGEMM_MID")
+    tuning("FT_FAIL_SCRATCH", 1)
+    unsplit = ft.qgemm_perchannel(at, 0.017, bt, sb, out_dtype=torch.bfloat16)
+    assert torch.equal(y, before) and torch.equal(y, unsplit)
+
+
 @pytest.mark.parametrize("m,n,k", GEMM_SHAPES)
 def test_qgemm_bit_exact(m, n, k):
     rng = np.random.default_rng(m * 1000 + n + k)
