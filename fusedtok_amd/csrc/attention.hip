@@ -1674,16 +1674,24 @@ int attention_run(const T* q, const T* k, const T* v, const int* table,
         // a bounded workspace that only the general kernel's partials fit
         const bool half128 = !std::is_same<T, float>::value && dim == kMfmaDim;
         if (half128 || bytes <= wsp.sure() || gen_bytes > wsp.sure()) {
-            char* ws = (char*)wsp.get(bytes, s);
-            if (dim == kMfmaDim)
+            char* ws = nullptr;
+            try {
+                ws = (char*)wsp.get(bytes, s);
+            } catch (const Error& err) {
+                // no room (or a capture before the shape's first call): the
+                // general kernel may need less
+                if (err.code != FT_EHIP || half128 || ap.k_new) throw;
+            }
+            if (ws && dim == kMfmaDim)
                 return attention_stream_run<T, 128>(
                     q, k, v, table, lens, out, batch, hq, hkv, rows_or_page, page_shift,
                     tbl_width, paged, (int)span, scale_log2, nseg, min_seg, low_seg, cus, ws, s,
                     amax, qcodes, qscale, ap);
-            return attention_stream_run<T, 64>(
-                q, k, v, table, lens, out, batch, hq, hkv, rows_or_page, page_shift, tbl_width,
-                paged, (int)span, scale_log2, nseg, min_seg, low_seg, cus, ws, s, amax, qcodes,
-                qscale, ap);
+            if (ws)
+                return attention_stream_run<T, 64>(
+                    q, k, v, table, lens, out, batch, hq, hkv, rows_or_page, page_shift,
+                    tbl_width, paged, (int)span, scale_log2, nseg, min_seg, low_seg, cus, ws, s,
+                    amax, qcodes, qscale, ap);
         }
     }
     if (ap.k_new) inval("attention: the append form runs on the stream kernel only");
@@ -1812,9 +1820,13 @@ void attention_append_run(const T* q, T* k_pool, T* v_pool, const int* table, co
         ap.v_new = v_new;
         ap.k_pool = k_pool;
         ap.v_pool = v_pool;
-        attention_run<T>(q, k_pool, v_pool, table, lens, out, batch, hq, hkv, page, tbl_width,
-                         dim, true, s, Workspace{}, nullptr, nullptr, nullptr, ap);
-        return;
+        try {
+            attention_run<T>(q, k_pool, v_pool, table, lens, out, batch, hq, hkv, page, tbl_width,
+                             dim, true, s, Workspace{}, nullptr, nullptr, nullptr, ap);
+            return;
+        } catch (const Error& err) {  // no workspace: the two ops may need less
+            if (err.code != FT_EHIP || dim == kMfmaDim) throw;
+        }
     }
     kv_append_run<T>(k_new, v_new, table, lens, k_pool, v_pool, batch, hkv, dim, page,
                      tbl_width, true, s);
