@@ -475,8 +475,13 @@ struct RmsqIo {
 // C4's 64 rows the two forms measured the same (layer 434.6-438.3 against
 // 437.4-438.7 us): the kernel boundary a graph replay pays costs about the
 // three dependent device-scope atomic round trips of grid_max.
+// Up to 64: the arrivals meet on one counter, one after the other (cols =
+// 4096, bf16 with a residual, graph replays, one launch against two: 64 rows
+// 6.4 / 6.0 us, 128 7.3 / 6.2, 256 9.0 / 7.0, 1000 29.5 / 13.6, 2048 97 / 22;
+// the layer's folded form at 64 rows gains from not storing its input).
 constexpr int kRmsqGridMinRows = 17;
-constexpr int kRmsqGridRows = 4096;
+constexpr int kRmsqGridRows = 64;
+constexpr int kRmsqGridMost = 4096;  // where there is no room for the row statistics
 
 // instantiates the row kernel K<T, RES, FK, FRES, HOUT> for the run-time
 // choices and calls launch(kernel pointer) with it
@@ -523,8 +528,17 @@ void rmsq_rows_run(const T* x, const RmsqIo<T>& io, const float* w, const T* r,
     const bool fres = fold && io.fold.res;
     const bool hout = r && io.h_out;
     if (fres && r) inval("rmsnorm_quant: a fold residual and a norm residual together");
-    if (cols <= 4 * kFNT * kRowChunks && rows >= kRmsqGridMinRows && rows <= kRmsqGridRows &&
-        tune(Tune::RmsqSplit, 0) == 0) {
+    const bool can_grid = cols <= 4 * kFNT * kRowChunks && rows >= kRmsqGridMinRows &&
+                          rows <= kRmsqGridMost && tune(Tune::RmsqSplit, 0) == 0;
+    RowStat* stat = nullptr;
+    if (!can_grid || rows > kRmsqGridRows) {
+        try {
+            stat = (RowStat*)scratch(Scratch::QuantMax, (size_t)rows * sizeof(RowStat), s);
+        } catch (const Error& err) {
+            if (err.code != FT_EHIP || !can_grid) throw;
+        }
+    }
+    if (!stat) {
         const GridMax gm = gridmax_state(rows, s);
         bool done = false;
         rmsq_pick<T, GridK>(r != nullptr, fk, fres, hout, [&](auto k) {
@@ -539,7 +553,7 @@ void rmsq_rows_run(const T* x, const RmsqIo<T>& io, const float* w, const T* r,
         if (done) return;
     }
     if (fold && !io.x_out) inval("rmsnorm_quant: the folded rows need a destination");
-    RowStat* stat = (RowStat*)scratch(Scratch::QuantMax, (size_t)rows * sizeof(RowStat), s);
+    if (!stat) stat = (RowStat*)scratch(Scratch::QuantMax, (size_t)rows * sizeof(RowStat), s);
     rmsq_pick<T, RowsK>(r != nullptr, fk, fres, hout, [&](auto k) {
         decltype(k)::fn<<<(unsigned)rows, kFNT, 0, s>>>(x, r, w, stat, cols, eps, io.fold,
                                                         io.x_out, io.h_out);
