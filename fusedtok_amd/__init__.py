@@ -68,6 +68,7 @@ from ._contract import Arr as _Arr
 from ._contract import Contract as _Contract
 from ._contract import Idx as _Idx
 from ._contract import Rule as _Rule
+from ._contract import current_stream as _stream
 from . import _sampling_args as _sargs
 
 __version__ = "0.1.0"
@@ -114,12 +115,14 @@ _CODE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 _SUFFIX = {torch.float32: "", torch.bfloat16: "_bf16", torch.float16: "_fp16"}
 
 
+_NATIVE = {}  # (entry, storage type) -> pybind function
+
+
 def _native(entry, dtype):
-    return getattr(_fusedtok, entry + _SUFFIX[dtype])
-
-
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    fn = _NATIVE.get((entry, dtype))
+    if fn is None:
+        fn = _NATIVE[entry, dtype] = getattr(_fusedtok, entry + _SUFFIX[dtype])
+    return fn
 
 
 def _out_dtype(out_dtype):
@@ -768,7 +771,10 @@ def rmsnorm_qgemm(x, weight, b_q, b_scales, *, residual=None, eps=1e-6, out_dtyp
     c = _RMS_QGEMM.bind(x=x, weight=weight, b_q=b_q, residual=residual)
     sb_ptr, sb = None, 0.0
     if torch.is_tensor(b_scales) or isinstance(b_scales, (list, tuple, np.ndarray)):
-        vec = torch.as_tensor(b_scales, dtype=torch.float32, device=c.device).contiguous()
+        vec = b_scales
+        if not (torch.is_tensor(vec) and vec.device == c.device and vec.dtype is torch.float32
+                and vec.is_contiguous()):
+            vec = torch.as_tensor(vec, dtype=torch.float32, device=c.device).contiguous()
         if vec.ndim != 1 or vec.numel() != c.N:
             raise ValueError("b_scales must be 1-D with N entries")
         b_scales = vec

@@ -143,6 +143,13 @@ class Rule:
         self.exc = exc
 
 
+def current_stream():
+    """The current torch stream's handle on the current device, as an int
+    (torch.cuda.current_stream().cuda_stream without building the Stream
+    object: 0.3 against 2 us)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def _parse(shape):
     if shape == "*" or shape.startswith("="):
         return shape
@@ -158,8 +165,7 @@ class Call:
         self._primary = values[contract.operands[0].name]
         self.device = device
         self.dims = {}
-        for k, v in values.items():
-            setattr(self, k, v)
+        self.__dict__.update(values)
 
     def __getattr__(self, name):
         dims = self.__dict__.get("dims", {})
@@ -211,6 +217,32 @@ class Call:
         return back(res)
 
 
+class _Plan:
+    """One operand of a contract, its strings parsed once for bind's device
+    path: ``syms`` is None for any shape, an operand's name for the shape of
+    that operand, or the tuple of shape symbols (``optional_first``: the
+    leading one may be missing)."""
+
+    def __init__(self, spec):
+        self.spec = spec
+        self.name = spec.name
+        self.arr = isinstance(spec, Arr)
+        self.optional = spec.optional
+        pat = _parse(spec.shape)
+        self.optional_first = False
+        if pat == "*":
+            self.syms = None
+        elif isinstance(pat, str):
+            self.syms = pat[1:]
+        else:
+            self.optional_first = bool(pat) and pat[0].endswith("?")
+            self.syms = (pat[0][:-1],) + pat[1:] if self.optional_first else pat
+        # a shape with a fixed size in it takes the general routine
+        self.fixed = isinstance(self.syms, tuple) and any(x.isdigit() for x in self.syms)
+        self.dtypes = spec.dtypes if self.arr else None
+        self.same_dtype = spec.same_dtype if self.arr else None
+
+
 class Contract:
     """The operands and rules of one op (module docstring). The first
     operand decides the path: a GPU tensor there means every operand must
@@ -223,14 +255,18 @@ class Contract:
         self.host_rules = host_rules
         self.rank_msg = rank_msg
         self.host = host
+        self._plans = tuple(_Plan(spec) for spec in operands)
+        self._first = operands[0].name
 
     def bind(self, **values):
-        primary = values[self.operands[0].name]
+        primary = values[self._first]
         gpu = torch.is_tensor(primary) and primary.is_cuda
+        if gpu:
+            return self._bind_device(values, primary)
         if not gpu and not self.host:
             raise TypeError(f"{self.operands[0].name} must be a GPU tensor (this op "
                             "has no host path)")
-        call = Call(self, values, primary.device if gpu else None)
+        call = Call(self, values, None)
         shapes = {}
         for spec in self.operands:
             v = values.get(spec.name)
@@ -239,18 +275,66 @@ class Contract:
                     raise TypeError(f"{spec.name} is required")
                 continue
             if isinstance(spec, Arr):
-                v = spec.on_device(v) if gpu else spec.on_host(v)
-                if spec.same_dtype is not None and gpu:
-                    other = getattr(call, spec.same_dtype)
-                    if v.dtype is not other.dtype:
-                        raise TypeError(f"{spec.name} must have the same dtype as "
-                                        f"{spec.same_dtype}")
+                v = spec.on_host(v)
                 self._bind_shape(call, spec, tuple(v.shape), shapes)
             else:
-                v = self._index(call, spec, v, gpu, shapes)
+                v = self._index(call, spec, v, False, shapes)
             setattr(call, spec.name, v)
             call._values[spec.name] = v
-        for rule in self.rules + (() if gpu else self.host_rules):
+        for rule in self.rules + self.host_rules:
+            if not rule.test(call):
+                raise rule.exc(rule.message)
+        return call
+
+    def _bind_device(self, values, primary):
+        """bind for a GPU primary operand: the common case of each check
+        inline (a short call's time is mostly here), the general routine -
+        which words the error or converts the operand - for the rest. Checks
+        run in the same order as on the host path."""
+        call = Call(self, values, primary.device)
+        attrs, dims, shapes = call.__dict__, call.dims, {}
+        for plan in self._plans:
+            name = plan.name
+            v = values.get(name)
+            if v is None:
+                if not plan.optional:
+                    raise TypeError(f"{name} is required")
+                continue
+            if not plan.arr:
+                if (isinstance(v, torch.Tensor) and v.is_cuda and v.dtype is torch.int32
+                        and v.is_contiguous()):
+                    self._bind_index_shape(call, plan.spec, v.shape, plan.syms)
+                else:
+                    attrs[name] = self._index(call, plan.spec, v, True, shapes)
+                continue
+            if not (isinstance(v, torch.Tensor) and v.is_cuda and v.dtype in plan.dtypes
+                    and v.is_contiguous()):
+                attrs[name] = v = plan.spec.on_device(v)
+            if plan.same_dtype is not None and v.dtype is not attrs[plan.same_dtype].dtype:
+                raise TypeError(f"{name} must have the same dtype as {plan.same_dtype}")
+            shape = shapes[name] = v.shape
+            syms = plan.syms
+            if syms is None:
+                continue
+            if isinstance(syms, str):
+                if shape != shapes[syms]:
+                    self._bind_shape(call, plan.spec, tuple(shape), shapes)
+                continue
+            if plan.optional_first and len(shape) == len(syms) - 1:
+                shape = (1,) + tuple(shape)
+            if len(shape) != len(syms) or plan.fixed:
+                self._bind_shape(call, plan.spec, tuple(v.shape), shapes)
+                continue
+            for sym, n in zip(syms, shape):
+                if sym in dims:
+                    if dims[sym] != n:
+                        raise ValueError(plan.spec.mismatch or
+                                         f"{name} has the wrong size in {sym}")
+                else:
+                    dims[sym] = n
+        for sym, n in dims.items():  # plain attributes (an operand's name wins)
+            attrs.setdefault(sym, n)
+        for rule in self.rules:
             if not rule.test(call):
                 raise rule.exc(rule.message)
         return call
@@ -298,8 +382,8 @@ class Contract:
         spec.check_range(host, call)
         return torch.from_numpy(host).to(call.device) if gpu else host
 
-    def _bind_index_shape(self, call, spec, shape):
-        syms = spec.shape.split()
+    def _bind_index_shape(self, call, spec, shape, syms=None):
+        syms = syms or spec.shape.split()
         ok = len(shape) == len(syms)
         if ok:
             for sym, n in zip(syms, shape):

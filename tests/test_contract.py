@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import fusedtok_amd as ft
+from fusedtok_amd import _contract as _contract_mod
 from fusedtok_amd import _sampling_args as sa
 from fusedtok_amd._contract import Arr, Contract, Idx, Rule
 
@@ -140,3 +141,93 @@ def test_history_forms_give_one_csr_layout():
     np.testing.assert_array_equal(sa.history_1d([5, 0], 6, None), [5, 0])
     with pytest.raises(ValueError, match=r"\[0, 6\)"):
         sa.history_1d([6], 6, None)
+
+
+class _DeviceTensor(torch.Tensor):
+    """A CPU tensor that says it is on the GPU: bind only looks at it."""
+    is_cuda = property(lambda self: True)
+
+
+def _dev(*shape, dtype=torch.float32):
+    return torch.zeros(shape, dtype=dtype).as_subclass(_DeviceTensor)
+
+
+def _bind_by_the_general_routines(contract, values):
+    """Contract.bind for device operands, every check through the general
+    routine of its operand."""
+    call = _contract_mod.Call(contract, dict(values), values[contract.operands[0].name].device)
+    shapes = {}
+    for spec in contract.operands:
+        v = values.get(spec.name)
+        if v is None:
+            if not spec.optional:
+                raise TypeError(f"{spec.name} is required")
+            continue
+        if isinstance(spec, Arr):
+            v = spec.on_device(v)
+            if spec.same_dtype is not None:
+                if v.dtype is not getattr(call, spec.same_dtype).dtype:
+                    raise TypeError(f"{spec.name} must have the same dtype as {spec.same_dtype}")
+            contract._bind_shape(call, spec, tuple(v.shape), shapes)
+        else:
+            v = contract._index(call, spec, v, True, shapes)
+        setattr(call, spec.name, v)
+    for rule in contract.rules:
+        if not rule.test(call):
+            raise rule.exc(rule.message)
+    return call
+
+
+_HALF = torch.bfloat16
+_PAGED = dict(q=_dev(2, 8, 64), k_pool=_dev(9, 2, 16, 64), v_pool=_dev(9, 2, 16, 64),
+              block_table=_dev(2, 4, dtype=torch.int32), lens=_dev(2, dtype=torch.int32))
+_NORM = dict(x=_dev(3, 8), weight=_dev(8), residual=_dev(3, 8))
+
+
+@pytest.mark.parametrize("contract,base,change", [
+    ("_DECODE_PAGED", _PAGED, {}),
+    ("_DECODE_PAGED", _PAGED, dict(lens=None)),
+    ("_DECODE_PAGED", _PAGED, dict(q=_dev(2, 8))),                      # rank
+    ("_DECODE_PAGED", _PAGED, dict(k_pool=_dev(9, 2, 16, 32))),         # D differs
+    ("_DECODE_PAGED", _PAGED, dict(v_pool=_dev(9, 2, 8, 64))),          # not k_pool's shape
+    ("_DECODE_PAGED", _PAGED, dict(k_pool=_dev(9, 2, 16, 64, dtype=_HALF))),   # storage type
+    ("_DECODE_PAGED", _PAGED, dict(q=_dev(2, 8, 64, dtype=torch.float64))),
+    ("_DECODE_PAGED", _PAGED, dict(q=_dev(2, 64, 8).transpose(1, 2))),  # not contiguous
+    ("_DECODE_PAGED", _PAGED, dict(k_pool=np.zeros((9, 2, 16, 64), np.float32))),
+    ("_DECODE_PAGED", _PAGED, dict(k_pool=torch.zeros(9, 2, 16, 64))),  # a CPU tensor
+    ("_DECODE_PAGED", _PAGED, dict(v_pool=None)),                       # required
+    ("_DECODE_PAGED", _PAGED, dict(lens=_dev(3, dtype=torch.int32))),
+    ("_DECODE_PAGED", _PAGED, dict(lens=_dev(2, dtype=torch.int64))),   # converted
+    ("_DECODE_PAGED", _PAGED, dict(lens=[1, 2])),                       # uploaded
+    ("_DECODE_PAGED", _PAGED, dict(lens=[1, 65])),                      # out of range
+    ("_DECODE_PAGED", _PAGED, dict(lens=np.array([0.5, 1.0]))),
+    ("_DECODE_PAGED", _PAGED, dict(block_table=_dev(8, dtype=torch.int32))),
+    ("_DECODE_PAGED", _PAGED, dict(block_table=_dev(4, 2, dtype=torch.int32).t())),
+    ("_DECODE_PAGED", _PAGED, dict(q=_dev(2, 6, 64))),                  # a rule: the group
+    ("_RMSNORM", _NORM, {}),
+    ("_RMSNORM", _NORM, dict(residual=None)),
+    ("_RMSNORM", _NORM, dict(x=_dev(8), residual=_dev(8))),             # no leading dimension
+    ("_RMSNORM", _NORM, dict(x=_dev(1, 3, 8))),
+    ("_RMSNORM", _NORM, dict(residual=_dev(3, 4))),
+    ("_RMSNORM", _NORM, dict(weight=_dev(9))),
+    ("_RMSNORM", _NORM, dict(weight=_dev(8, dtype=_HALF))),             # converted
+    ("_RMSNORM", _NORM, dict(weight=_dev(16)[::2])),                    # made contiguous
+    ("_RMSNORM", _NORM, dict(x=_dev(3, 0), weight=_dev(0), residual=None)),  # a rule
+])
+def test_device_binding_equals_the_general_routines(contract, base, change):
+    # bind's inline checks for device operands against the operands' general
+    # routines, over every form they tell apart: the same symbols and
+    # operands, or the same error
+    contract = getattr(ft, contract)
+
+    def outcome(bind):
+        try:
+            call = bind({**base, **change})
+        except (TypeError, ValueError) as exc:
+            return type(exc), str(exc)
+        ops = {s.name: getattr(call, s.name) for s in contract.operands}
+        return dict(call.dims), {k: None if v is None else (tuple(v.shape), v.dtype, v.is_contiguous())
+                                 for k, v in ops.items()}, call.on_gpu
+
+    got = outcome(lambda values: contract.bind(**values))
+    assert got == outcome(lambda values: _bind_by_the_general_routines(contract, values))
