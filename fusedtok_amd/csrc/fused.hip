@@ -469,17 +469,17 @@ struct RmsqIo {
     bool store_x = true;  // false: the one-launch form need not store x_out
 };
 
-// Rows (workgroups) of the one-launch form. From 17 rows: below, the two
-// launches measured as fast or faster (C2 chain, M = 8 / 16, same box:
-// 15.74 / 16.35 us with two launches against 15.80 / 16.60 with one); at
-// C4's 64 rows the two forms measured the same (layer 434.6-438.3 against
-// 437.4-438.7 us): the kernel boundary a graph replay pays costs about the
-// three dependent device-scope atomic round trips of grid_max.
+// Rows (workgroups) of the one-launch form. From 5 rows (rmsq_small takes
+// fewer): in a graph replay the two forms measure the same (5 x 2048 bf16
+// 5.0 us with one launch, 5.3 with two; 16 x 4096 5.7 / 5.6; C4's layer at 64
+// rows 434.6-438.3 against 437.4-438.7: the kernel boundary a replay pays
+// costs about the three dependent device-scope atomic round trips of
+// grid_max), and an eager call saves a launch (10.6 against 13.3 us).
 // Up to 64: the arrivals meet on one counter, one after the other (cols =
 // 4096, bf16 with a residual, graph replays, one launch against two: 64 rows
 // 6.4 / 6.0 us, 128 7.3 / 6.2, 256 9.0 / 7.0, 1000 29.5 / 13.6, 2048 97 / 22;
 // the layer's folded form at 64 rows gains from not storing its input).
-constexpr int kRmsqGridMinRows = 17;
+constexpr int kRmsqGridMinRows = 5;
 constexpr int kRmsqGridRows = 64;
 constexpr int kRmsqGridMost = 4096;  // where there is no room for the row statistics
 
@@ -516,6 +516,19 @@ struct GridK {
     static constexpr auto fn = rmsq_grid<T, RES, FK, FRES, HOUT>;
 };
 
+// grid_max state for nwg workgroups, or false where there is no room for it
+// (a capture before the first call, an allocation that fails): the step then
+// takes its two launches
+bool grid_room(int nwg, hipStream_t s, GridMax& gm) {
+    try {
+        gm = gridmax_state(nwg, s);
+        return true;
+    } catch (const Error& err) {
+        if (err.code != FT_EHIP) throw;
+        return false;
+    }
+}
+
 // rmsnorm_quant of x (or of the folded partials) in one launch when every
 // row's workgroup can be resident at once, else the row pass then the fold
 // of the row maxima and the codes (two launches)
@@ -538,8 +551,8 @@ void rmsq_rows_run(const T* x, const RmsqIo<T>& io, const float* w, const T* r,
             if (err.code != FT_EHIP || !can_grid) throw;
         }
     }
-    if (!stat) {
-        const GridMax gm = gridmax_state(rows, s);
+    GridMax gm{};
+    if (!stat && grid_room(rows, s, gm)) {
         bool done = false;
         rmsq_pick<T, GridK>(r != nullptr, fk, fres, hout, [&](auto k) {
             using Kt = decltype(k);
@@ -709,6 +722,40 @@ __global__ __launch_bounds__(kFNT) void swq_quant(
     }
 }
 
+// Both passes in one launch for a step's few elements (4 a thread): the
+// maximum folded with grid_max, the codes from the registers. Every workgroup
+// resident at once, at most kSwqGridWgs of them: from there the arrivals on
+// the one counter cost a graph replay more than the second launch (bf16, one
+// launch against two, us: 4 x 2816, 11 workgroups, 5.1 / 5.5; 6 x 8192, 48,
+// 5.6 / 5.7; 8 x 8192, 64, 5.9 / 5.6); an eager call saves 2.8 us of host time.
+constexpr int kSwqGridWgs = 48;
+
+template <typename T>
+__global__ __launch_bounds__(kFNT) void swq_grid(
+    const T* __restrict__ g, const T* __restrict__ u, signed char* __restrict__ q,
+    float* __restrict__ scale_out, int rows, int cols, long long ld, GridMax gm) {
+    __shared__ float red[kFNT / 64];
+    const long long c = (long long)blockIdx.x * kFNT + threadIdx.x;
+    const bool live = c < (long long)rows * cols / 4;
+    float y[4] = {0.f, 0.f, 0.f, 0.f};
+    if (live) swq_at<T, true>(g, u, c, cols, ld, y);
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m = fmaxf(m, fabsf(y[k]));
+    m = block_max<kFNT>(m, red);
+    m = grid_max<kFNT>(gm, m, red);
+    const float scale = make_scale(m);
+    const float inv_s = 1.0f / scale;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
+    if (!live) return;
+    char4 o;
+    o.x = quant1(y[0], inv_s);
+    o.y = quant1(y[1], inv_s);
+    o.z = quant1(y[2], inv_s);
+    o.w = quant1(y[3], inv_s);
+    *reinterpret_cast<char4*>(q + 4 * c) = o;
+}
+
 constexpr int kSwqParts = 1024;
 
 template <typename T>
@@ -722,6 +769,15 @@ void swiglu_quant_run(const T* g, const T* u, signed char* q, float* scale_out,
     const bool vec = cols % 4 == 0 && ld % 4 == 0 && (uintptr_t)g % a4 == 0 &&
                      (uintptr_t)u % a4 == 0 && (uintptr_t)q % 4 == 0;
     const long long n = (long long)rows * cols / (vec ? 4 : 1);
+    const long long wgs = (n + kFNT - 1) / kFNT;
+    GridMax gm{};
+    if (vec && wgs <= kSwqGridWgs && grid_room((int)wgs, s, gm)) {
+        if (grid_resident((const void*)swq_grid<T>, (int)wgs, kFNT, GridUse::SwiGLU)) {
+            swq_grid<T><<<(unsigned)wgs, kFNT, 0, s>>>(g, u, q, scale_out, rows, cols, ld, gm);
+            launch_check("swiglu_quant one-launch kernel launch");
+            return;
+        }
+    }
     float* part = (float*)scratch(Scratch::QuantMax, kSwqParts * sizeof(float), s);
     const unsigned g1 = grid_1d(n, kFNT, kSwqParts);
     const unsigned g2 = grid_1d(n, kFNT, dev_info().cu_count * 4);

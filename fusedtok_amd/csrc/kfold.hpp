@@ -33,10 +33,13 @@ struct KFold {
 // int32 partials are left in the library's GEMM scratch, `f` describes them
 // and the result is true: the caller's next launch on stream s must fold
 // them (before any other GEMM reuses that scratch). Otherwise y is written
-// and the result is false. qgemm.hip.
+// and the result is false; a residual `res` [m, n] (y's type) is then added
+// to it as residual_add does where the kernel's epilogue can (M <= 16), and
+// *res_done says so. qgemm.hip.
 bool qgemm_deferred(const signed char* a, const signed char* b, const float* sa_dev,
                     const float* sb_vec, void* y, int y_dtype, int m, int n, int k,
-                    hipStream_t s, KFold& f);
+                    hipStream_t s, KFold& f, const void* res = nullptr,
+                    bool* res_done = nullptr);
 
 // The gate/up GEMM of swiglu_quant: y [m, 2 inter] = A . B^T as
 // ft_qgemm_launch_ex writes it (B: inter gate rows, then inter up rows).

@@ -147,9 +147,12 @@ void forward(ft_decode_layer& L, const Args& a, hipStream_t s, const HandIn* in 
     qgemm_swiglu_quant_codes(d.dtype, L.q2, s2, d.w_gu, d.s_gu, L.h, L.q3, s3, B, d.inter,
                              d.hidden, s);
     // down GEMM + the residual stream: folded with the K-split partials (by
-    // the next layer's first row pass in a stack), else added in place
+    // the next layer's first row pass in a stack), added by the GEMM's
+    // epilogue, or in place behind it
     KFold f;
-    if (qgemm_deferred(L.q3, d.w_down, s3, d.s_down, a.y, d.dtype, B, d.hidden, d.inter, s, f)) {
+    bool added = false;
+    if (qgemm_deferred(L.q3, d.w_down, s3, d.s_down, a.y, d.dtype, B, d.hidden, d.inter, s, f,
+                       L.res, &added)) {
         f.res = L.res;
         if (defer)
             *defer = f;
@@ -157,7 +160,7 @@ void forward(ft_decode_layer& L, const Args& a, hipStream_t s, const HandIn* in 
             kfold_store(f, a.y, d.dtype, B, s);
     } else {
         if (defer) *defer = KFold{};
-        residual_add(d.dtype, a.y, L.res, (long long)B * d.hidden, s);
+        if (!added) residual_add(d.dtype, a.y, L.res, (long long)B * d.hidden, s);
     }
 }
 

@@ -97,6 +97,9 @@ struct Epi {
     const float* sa_dev;  // device scale overrides sa when non-null
     float sb;
     const float* sb_vec;  // per-channel scales, null = per-tensor sb
+    // (decode kernels) an output-typed [m, n] added to the stored value and
+    // rounded again: a decode layer's residual add (kfold.hpp)
+    const void* res = nullptr;
 };
 
 __device__ __forceinline__ float epi_sa(const Epi& e) {
@@ -171,6 +174,25 @@ __device__ __forceinline__ void epi_store(const Epi& e, float sa, int n,
     float s = 0.0f;
     if constexpr (OUT != kOutI32) s = e.sb_vec ? sa * e.sb_vec[col] : sa * e.sb;
     epi_store_scaled<OUT>(e, n, row, col, acc, s);
+}
+
+// epi_store with e.res, where there is one (the decode kernels)
+template <int OUT>
+__device__ __forceinline__ void epi_store_res(const Epi& e, float sa, int n,
+                                              int row, int col, int acc) {
+    if constexpr (OUT != kOutI32) {
+        if (e.res) {
+            using T = std::conditional_t<OUT == kOutBF16, bf16,
+                                         std::conditional_t<OUT == kOutF16, f16, float>>;
+            const size_t idx = (size_t)row * n + col;
+            const float s = e.sb_vec ? sa * e.sb_vec[col] : sa * e.sb;
+            const float v = kfold_add_res<T>(epi_stored<OUT>(acc, s),
+                                             St<T>::ld(static_cast<const T*>(e.res) + idx));
+            St<T>::st(static_cast<T*>(e.y) + idx, v);
+            return;
+        }
+    }
+    epi_store<OUT>(e, sa, n, row, col, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -277,7 +299,7 @@ __global__ __launch_bounds__(256) void qgemv_dot4(const i8* __restrict__ a,
 #pragma unroll
             for (int mm = 0; mm < M_; ++mm)
                 if (lane == r * M_ + mm && j0 + r < n)
-                    epi_store<OUT>(e, sa, n, mm, j0 + r, acc[r][mm]);
+                    epi_store_res<OUT>(e, sa, n, mm, j0 + r, acc[r][mm]);
     }
 }
 
@@ -533,7 +555,7 @@ __global__ __launch_bounds__(64 * KW) void qgemm_dec(
     const float sa = epi_sa(e);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        if (4 * g + i < m) epi_store<OUT>(e, sa, n, 4 * g + i, col, acc[i]);
+        if (4 * g + i < m) epi_store_res<OUT>(e, sa, n, 4 * g + i, col, acc[i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -642,7 +664,7 @@ __global__ __launch_bounds__(64) void qgemm_dec_lds(
     const float sa = epi_sa(e);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        if (4 * g + i < m) epi_store<OUT>(e, sa, n, 4 * g + i, col, acc[i]);
+        if (4 * g + i < m) epi_store_res<OUT>(e, sa, n, 4 * g + i, col, acc[i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -2339,8 +2361,9 @@ bool qgemm_mid_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, in
 }
 
 template <int OUT>
-void qgemm_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, int k,
-                    hipStream_t s, KFold* defer) {
+void qgemm_dispatch(const i8* a, const i8* b, const Epi& e0, int m, int n, int k,
+                    hipStream_t s, KFold* defer, const void* res, bool* res_done) {
+    Epi e = e0;
     const bool aligned = (k % 16 == 0) && ((uintptr_t)a % 16 == 0) &&
                          ((uintptr_t)b % 16 == 0);
     // FT_QGEMM_KERNEL: 1 skinny, 2 tiled, 3 scalar, 4 big, 5 gemv, 6 decode
@@ -2359,6 +2382,8 @@ void qgemm_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, int k,
     // 14.0 us vs 37.1 us).
     if ((m == 1 && force == 0) || force == 5) {
         if (m > 8) inval("gemv qgemm supports m <= 8");
+        e.res = res;
+        if (res_done) *res_done = res != nullptr;
         const long long waves = std::min<long long>((n + kGemvRows - 1) / kGemvRows,
                                                     (long long)dev_info().cu_count * 16);
         const unsigned grid = (unsigned)((waves + 3) / 4);
@@ -2377,6 +2402,8 @@ void qgemm_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, int k,
     }
     if ((m <= 16 && force == 0) || force == 6) {
         if (m > 16) inval("decode qgemm supports m <= 16");
+        e.res = res;
+        if (res_done) *res_done = res != nullptr;
         const int tiles = (n + 15) / 16;
         const unsigned grid = (unsigned)tiles;
         // waves per 16-column tile: one long stream per wave when there are
@@ -2523,8 +2550,11 @@ void qgemm_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, int k,
     launch_check("qgemm tiled kernel launch");
 }
 
+// res (output-typed [m, n], or null): added to the output where the kernel
+// can (res_done), as residual_add would after it.
 void qgemm_run(const i8* a, const i8* b, Epi e, int out, int m, int n, int k,
-               hipStream_t s, KFold* defer = nullptr) {
+               hipStream_t s, KFold* defer = nullptr, const void* res = nullptr,
+               bool* res_done = nullptr) {
     qgemm_check(m, n, k);
     if (m == 0 || n == 0) return;
     if (!e.y) inval("qgemm: null output");
@@ -2536,10 +2566,10 @@ void qgemm_run(const i8* a, const i8* b, Epi e, int out, int m, int n, int k,
     }
     if (!a || !b) inval("qgemm: null operand");
     switch (out) {
-    case kOutF32: qgemm_dispatch<kOutF32>(a, b, e, m, n, k, s, defer); break;
-    case kOutBF16: qgemm_dispatch<kOutBF16>(a, b, e, m, n, k, s, defer); break;
-    case kOutF16: qgemm_dispatch<kOutF16>(a, b, e, m, n, k, s, defer); break;
-    case kOutI32: qgemm_dispatch<kOutI32>(a, b, e, m, n, k, s, defer); break;
+    case kOutF32: qgemm_dispatch<kOutF32>(a, b, e, m, n, k, s, defer, res, res_done); break;
+    case kOutBF16: qgemm_dispatch<kOutBF16>(a, b, e, m, n, k, s, defer, res, res_done); break;
+    case kOutF16: qgemm_dispatch<kOutF16>(a, b, e, m, n, k, s, defer, res, res_done); break;
+    case kOutI32: qgemm_dispatch<kOutI32>(a, b, e, m, n, k, s, defer, res, res_done); break;
     default: inval("qgemm: unknown output type");
     }
 }
@@ -2636,7 +2666,7 @@ void kfold_store(const KFold& f, void* y, int dtype, int m, hipStream_t s) {
 
 bool qgemm_deferred(const signed char* a, const signed char* b, const float* sa_dev,
                     const float* sb_vec, void* y, int y_dtype, int m, int n, int k,
-                    hipStream_t s, KFold& f) {
+                    hipStream_t s, KFold& f, const void* res, bool* res_done) {
     if (!sa_dev || !sb_vec) inval("qgemm: a device scale and per-channel scales are required");
     int out;
     switch (y_dtype) {
@@ -2646,8 +2676,9 @@ bool qgemm_deferred(const signed char* a, const signed char* b, const float* sa_
     default: inval("qgemm: unknown output dtype code");
     }
     f = KFold{};
+    if (res_done) *res_done = false;
     Epi e{y, 0.0f, sa_dev, 0.0f, sb_vec};
-    qgemm_run(a, b, e, out, m, n, k, s, &f);
+    qgemm_run(a, b, e, out, m, n, k, s, &f, res, res_done);
     return f.ksplit > 1;
 }
 

@@ -673,3 +673,40 @@ def test_decode_layer_graph_replays_equal_eager():
         eager = layer()               # eager work between replays
         torch.cuda.synchronize()
         assert torch.equal(eager, ref)
+
+
+@pytest.mark.parametrize("dt", ALL)
+@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 260), (6, 8192), (48, 1024), (49, 1024),
+                                       (7, 1020)])
+def test_swiglu_quant_grid_launch_matches_two_launches(dt, rows, cols, tuning):
+    # up to 48 workgroups (4 elements a thread) swiglu_quant is one launch
+    # with the maximum folded inside it; FT_GRID_SYNC=2 forces the two. Eight
+    # calls back to back, the largest value in another place each time.
+    rng = np.random.default_rng(rows * 31 + cols)
+    hs = []
+    for i in range(8):
+        h = rng.standard_normal((rows, 2 * cols)).astype(np.float32)
+        h[i % rows, (i * 7) % cols] = 20.0 + i
+        h[i % rows, cols + (i * 7) % cols] = 3.0
+        hs.append(t(h, dt))
+    call = lambda h: ft.swiglu_quant(h[:, :cols], h[:, cols:], device_scale=True)  # noqa: E731
+    got = [call(h) for h in hs]
+    tuning("FT_GRID_SYNC", 2)
+    ref = [call(h) for h in hs]
+    for i, ((q1, s1), (q2, s2)) in enumerate(zip(got, ref)):
+        assert torch.equal(s1, s2) and torch.equal(q1, q2), f"call {i}"
+
+
+@pytest.mark.parametrize("dt", ALL)
+@pytest.mark.parametrize("rows,cols", [(5, 4096), (6, 12), (16, 2048), (65, 1028)])
+def test_rmsnorm_quant_few_rows_match_two_launches(dt, rows, cols, tuning):
+    # one launch from 5 rows to 64, two from 65; the same codes either way
+    rng = np.random.default_rng(rows + cols)
+    w = t(rng.uniform(0.5, 1.5, cols).astype(np.float32))
+    x, r = (t(rng.standard_normal((rows, cols)).astype(np.float32), dt) for _ in range(2))
+    for res in (None, r):
+        q1, s1 = ft.rmsnorm_quant(x, w, residual=res, eps=1e-5)
+        tuning("FT_RMSQ_SPLIT", 1)
+        q2, s2 = ft.rmsnorm_quant(x, w, residual=res, eps=1e-5)
+        tuning.clear("FT_RMSQ_SPLIT")
+        assert torch.equal(q1, q2) and s1 == s2

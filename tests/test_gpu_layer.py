@@ -344,3 +344,22 @@ def test_stack_max_batch_is_the_smallest_and_empty_batches():
     stack.close()
     big.close()
     small.close()
+
+
+@pytest.mark.parametrize("b", [1, 2, 9, 16, 17])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_small_batches_add_the_residual_in_the_gemm(b, dt):
+    # up to 16 rows the down GEMM's epilogue adds the residual stream (the
+    # GEMV at one row, the decode kernels above); 17 rows fold or add it
+    # behind. The layer and a stack of two equal the op chain.
+    cfg = dict(TOY, b=b, lens=[(37 * i) % 290 + 1 for i in range(b)])
+    w, x, kp, vp, table, lens = make_case(cfg, dt, 40 + b)
+    k_ref, v_ref = kp.clone(), vp.clone()
+    y_ref = op_chain(cfg, w, x, k_ref, v_ref, table, lens, dt)
+    layer = make_layer(cfg, w, dt)
+    y = layer(x, kp, vp, table, lens)
+    assert np.array_equal(raw(y), raw(y_ref))
+    k2, v2 = kp.clone(), vp.clone()
+    y2_ref = op_chain(cfg, w, y_ref, k_ref.clone(), v_ref.clone(), table, lens, dt)
+    y2 = ft.DecodeStack([layer, layer])(x, [kp, k2], [vp, v2], table, lens)
+    assert np.array_equal(raw(y2), raw(y2_ref))
