@@ -148,8 +148,9 @@ void* scratch_zeroed(Scratch which, size_t bytes, hipStream_t s);
 // Grid-wide maximum inside one launch (grid_max below). The state is one
 // 64-bit word (generation << 32 | arrivals) and one 32-bit slot per
 // workgroup, zeroed when allocated; every launch leaves the arrivals at 0.
-// Launches that use it are ordered on one stream: calls that overlap on one
-// GPU race, as with the library's other scratch.
+// Launches that use one state are ordered: a stream's launches share a state
+// and streams hash to 16 of them (calls that overlap on one GPU still race on
+// the library's other scratch).
 struct GridMax {
     unsigned long long* word;
     unsigned* slots;

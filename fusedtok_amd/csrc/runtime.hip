@@ -125,6 +125,9 @@ bool stream_capturing(hipStream_t s) {
 }
 
 namespace {
+constexpr int kGridStates = 16;
+constexpr int kGridMostWgs = 4096;  // workgroups per state
+
 void* scratch_impl(Scratch which, size_t bytes, hipStream_t s, bool zero) {
     // test hook, checked before any HIP call so that a host without a
     // device reaches it too
@@ -153,6 +156,8 @@ void* scratch_impl(Scratch which, size_t bytes, hipStream_t s, bool zero) {
     }
     if (zero) {
         e = hipMemsetAsync(p, 0, want, s);
+        // done before another stream's launch can use it
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) {
             (void)hipFree(p);
             hip_fail("device scratch clear", e);
@@ -173,15 +178,22 @@ void* scratch_zeroed(Scratch which, size_t bytes, hipStream_t s) {
 }
 
 GridMax gridmax_state(int nwg, hipStream_t s) {
-    // the word, then the slots from byte 256; zeroed when (re)allocated, and
-    // every launch leaves the arrivals at 0 (the generation keeps counting)
-    char* p = (char*)scratch_zeroed(Scratch::GridSync, 256 + 4 * (size_t)(nwg > 0 ? nwg : 1), s);
+    // kGridStates states of one size, each a word and, from byte 256, the
+    // slots; zeroed when allocated, and every launch leaves the arrivals at 0
+    // (the generation keeps counting). A stream takes the state its handle
+    // hashes to: launches of one stream are ordered, and those of two streams
+    // that overlap then hardly ever meet on one counter.
+    if (nwg > kGridMostWgs) nwg = kGridMostWgs;  // (more are never resident at once)
+    constexpr size_t kState = 256 + 4 * (size_t)kGridMostWgs;
+    char* p = (char*)scratch_zeroed(Scratch::GridSync, kGridStates * kState, s);
+    const unsigned long long h = (unsigned long long)(uintptr_t)s * 0x9E3779B97F4A7C15ull;
+    p += (h >> 60) % kGridStates * kState;
     return GridMax{(unsigned long long*)p, (unsigned*)(p + 256)};
 }
 
 bool grid_resident(const void* kernel, int nwg, int threads, GridUse use) {
     const int off = tune(Tune::GridSync, 0);
-    if (nwg < 1 || (off & 1) || (off & (int)use)) return false;
+    if (nwg < 1 || nwg > kGridMostWgs || (off & 1) || (off & (int)use)) return false;
     const int dev = current_device();
     const int cus = dev_info().cu_count;
     static std::mutex mu;
