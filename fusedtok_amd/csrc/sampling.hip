@@ -243,8 +243,12 @@ __device__ void select_prefix(const SampleRow& row, float vmax, u64 T, SmpShared
             // segment whose offsets enclose it
             const int total = sh.seg_off[pre.S];
             for (int j = tid; j < total; j += kSmpNT) {
-                int sg = 0;
-                while (sh.seg_off[sg + 1] <= j) ++sg;
+                // the last segment starting at or before j
+                int sg = 0, hi = pre.S - 1;
+                while (sg < hi) {
+                    const int mid = (sg + hi + 1) >> 1;
+                    if (sh.seg_off[mid] <= j) sg = mid; else hi = mid - 1;
+                }
                 const size_t at = (size_t)sg * pre.cap + (j - sh.seg_off[sg]);
                 // the mass is loaded with the key, not after the bin test:
                 // one memory round trip per query instead of two
@@ -536,10 +540,14 @@ __global__ __launch_bounds__(kSmpNT) void sample_topp_rows(
 //                      row scans, and a crossing bin beyond the exact sort's
 //                      capacity by the radix passes, as in sample_topp_rows
 // ---------------------------------------------------------------------------
-constexpr int kSliceNT = 256;
-constexpr int kMinSlice = 8192;    // tokens per slice at least
+// 1024 threads: the slice passes are a few loads, then ~25 instructions and an
+// LDS atomic a token, and 16 waves a workgroup hide each other's waits (64
+// rows of 128256 tokens, 8 slices: 79.7 us a call with 256 threads and 16
+// loads a thread, 67.0 with 512 and 8, 60.7 with 1024 and 4).
+constexpr int kSliceNT = 1024;
+constexpr int kMinSlice = 4096;    // tokens per slice at least
 constexpr int kSliceCap = 1024;    // gathered candidates per slice
-constexpr int kSliceLoads = 16;    // 16-byte loads in flight per thread: a
+constexpr int kSliceLoads = 4;     // 16-byte loads in flight per thread: a
                                    // 16k-token slice in one round trip
 // LDS bitmap words of one slice: the sliced path runs with S >= 2, so a
 // slice holds at most ceil(n / 2) + 31 tokens, n <= kMaxBitmapVocab
@@ -637,10 +645,11 @@ __global__ __launch_bounds__(kSliceNT) void smp_slice_max(SliceArgs a) {
     if (seed_lane) a.seedv[r] = seed;
 }
 
+// The row's maximum: lane s of every wave loads slice s's (S <= kMaxSlices =
+// 64), one round trip.
 __device__ __forceinline__ float row_max_of(const SliceArgs& a, int r) {
-    float vmax = -INFINITY;
-    for (int s = 0; s < a.S; ++s) vmax = fmaxf(vmax, a.smax[r * a.S + s]);
-    return vmax;
+    const int s = threadIdx.x & 63;
+    return wave_max(a.smax[r * a.S + min(s, a.S - 1)]);
 }
 
 __global__ __launch_bounds__(kSliceNT) void smp_slice_hist(SliceArgs a) {
@@ -979,24 +988,31 @@ void topp_launch(const float* x, int rows, int n, float p, float t, float pen,
     if (!x || !out) inval("sampling: null operand");
     if (penal && !ids) inval("sampling: null token ids");
     const float inv_t = 1.0f / t;  // the reference's order (inv_t = 1.0f / t)
-    // slices per row: enough workgroups for about two per CU, at least
-    // kMinSlice tokens each; FT_SMP_SINGLE=1 keeps one workgroup per row
+    // slices per row: a workgroup per CU, or more (up to two) while a slice
+    // is longer than one batch of loads; at least kMinSlice tokens each.
+    // us a call at S = 2 / 4 / 8 / 16 / 32: 64 x 128256 75 / 62 / 60 / 71 / 93,
+    // 16 x 128256 71 / 56 / 48 / 46 / 49, 1 x 128256 66 / 52 / 46 / 42 / 41,
+    // 128 x 50000 51 / 50 / 63 / 88 / 135, 16 x 32000 41 / 38 / 37 / 37 / 41.
+    // FT_SMP_SINGLE=1 keeps one workgroup per row
     const int cus = dev_info().cu_count;
     int S = 1;
-    if (rows < cus && tune(Tune::SmpSingle, 0) == 0)
-        S = std::min({(2 * cus + rows - 1) / rows, std::max(1, n / kMinSlice), kMaxSlices});
+    if (rows < cus && tune(Tune::SmpSingle, 0) == 0) {
+        constexpr int kBatch = 4 * kSliceLoads * kSliceNT;  // tokens
+        S = std::min({std::max(cus / rows, (n + kBatch - 1) / kBatch),
+                      std::max(1, 2 * cus / rows), std::max(1, n / kMinSlice), kMaxSlices});
+    }
     // FT_SMP_SLICES forces the slice count (2 .. kMaxSlices, at most one
     // slice per 32 tokens)
     const int forced_s = tune(Tune::SmpSlices, 0);
     if (forced_s >= 2 && tune(Tune::SmpSingle, 0) == 0)
         S = std::min({forced_s, kMaxSlices, std::max(1, n / 32)});
-    if (S <= 1) {
+    auto one_workgroup_per_row = [&] {
         sample_topp_rows<<<(unsigned)rows, kSmpNT, 0, s>>>(
             x, n, p, inv_t, pen, penal ? ids : nullptr, penal ? offs : nullptr, m, seeds, seed0,
             out);
         launch_check("sampling kernel launch");
-        return;
-    }
+    };
+    if (S <= 1) return one_workgroup_per_row();
     int slen = (n + S - 1) / S;
     slen = (slen + 31) & ~31;  // whole bitmap words, 16-byte aligned starts
     S = (n + slen - 1) / slen;
@@ -1028,7 +1044,13 @@ void topp_launch(const float* x, int rows, int n, float p, float t, float pen,
                  o_seed = take(R * 8),
                  o_gn = take(R * S * 4), o_gk = take(R * S * kSliceCap * 8),
                  o_gq = take(R * S * kSliceCap * 8);
-    char* ws = (char*)scratch(Scratch::Sampling, off, s);
+    char* ws = nullptr;
+    try {
+        ws = (char*)scratch(Scratch::Sampling, off, s);
+    } catch (const Error& err) {  // no room (or a capture before the first call)
+        if (err.code != FT_EHIP) throw;
+        return one_workgroup_per_row();
+    }
     a.bits = (unsigned*)(ws + o_bits);
     a.smax = (float*)(ws + o_smax);
     a.mhist = (u64*)(ws + o_mh);
