@@ -998,7 +998,7 @@ void topp_launch(const float* x, int rows, int n, float p, float t, float pen,
     int S = 1;
     if (rows < cus && tune(Tune::SmpSingle, 0) == 0) {
         constexpr int kBatch = 4 * kSliceLoads * kSliceNT;  // tokens
-        S = std::min({std::max(cus / rows, (n + kBatch - 1) / kBatch),
+        S = std::min({std::max(cus / rows, (n - 1) / kBatch + 1),
                       std::max(1, 2 * cus / rows), std::max(1, n / kMinSlice), kMaxSlices});
     }
     // FT_SMP_SLICES forces the slice count (2 .. kMaxSlices, at most one

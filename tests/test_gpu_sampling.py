@@ -229,6 +229,24 @@ def test_sliced_pipeline_matches_single_workgroup(rows, n, tuning):
         assert got[0] == got[1], (p, temp)
 
 
+@pytest.mark.parametrize("rows,n", [(1, 8191), (1, 8192), (2, 12289), (31, 16385), (200, 16384),
+                                    (200, 32769), (255, 8193)])
+def test_slice_count_rule_edges_match_single_workgroup(rows, n, tuning):
+    # where a row starts to be cut (two slices of 4096 tokens), slices just
+    # over one batch of loads (16384 tokens), and few CUs a row; with no room
+    # for the slices' workspace one workgroup takes each row
+    rng = np.random.default_rng(rows + n)
+    lt = t((rng.standard_normal((rows, n)) * 2).astype(np.float32))
+    seeds = list(range(rows))
+    call = lambda: ft.sample_topp_batched(lt, 0.9, temperature=0.8, seeds=seeds).tolist()  # noqa: E731
+    got = call()
+    tuning("FT_SMP_SINGLE", 1)
+    assert got == call()
+    tuning.clear("FT_SMP_SINGLE")
+    tuning("FT_FAIL_SCRATCH", 1)
+    assert got == call()
+
+
 @pytest.mark.parametrize("slices", [2, 3, 12, 64])
 def test_sliced_pipeline_any_slice_count(slices, tuning):
     # forced slice counts (FT_SMP_SLICES): odd splits, slices of a few
