@@ -137,12 +137,14 @@ int ft_attention_decode_paged_launch_fp16(const void* q, const void* k_pool,
 /* FT_NOALLOC_WORKSPACE_BYTES (16 MiB) instead of the library's growing */
 /* buffer, and no hipMalloc, hipFree or other allocating routine is     */
 /* called. A call whose partials do not fit returns FT_EINVAL before    */
-/* anything is launched. With D = 128 and G = q_heads / kv_heads <= 16  */
-/* the need is (2 * CUs + batch * kv_heads) * G * 520 + 8 * (batch + 2) */
-/* bytes: 1.6 MB for batch 32 with 32 / 8 heads on 256 CUs; batch 512   */
-/* at 32 / 8 heads still fits. Every call on one GPU shares that GPU's  */
-/* array, which keeps the last call's contents: calls that overlap on   */
-/* one GPU (unordered streams) race and must be serialised.             */
+/* anything is launched. With D = 64 or 128 and G = q_heads / kv_heads  */
+/* <= 16 the need is (2 * CUs + batch * kv_heads) * G * 4 * (D + 2) + 8 */
+/* * (batch + 2) bytes: at D = 128, 1.6 MB for batch 32 with 32 / 8     */
+/* heads on 256 CUs, and batch 512 still fits; at D = 64 a call that    */
+/* needs more runs where the general kernel's partials fit. Every call  */
+/* on one GPU shares that GPU's array, which keeps the last call's      */
+/* contents: calls that overlap on one GPU (unordered streams) race and */
+/* must be serialised.                                                  */
 #define FT_NOALLOC_WORKSPACE_BYTES (16u << 20)
 int ft_attention_decode_paged_launch_bf16_noalloc(const void* q, const void* k_pool,
                                                   const void* v_pool,
