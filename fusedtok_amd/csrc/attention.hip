@@ -787,9 +787,13 @@ void attn_decode_stream(
 // staging (32 rows x 128 B each; chunk c of row w at c ^ ((w >> 1) & 7), so
 // the 16 lanes of a write - two rows - and of a fragment read - 16 rows, one
 // chunk - hit 16 different 16-byte bank groups), K into the score MFMAs' A
-// operand, V through ds_read_b64_tr_b16 straight into the PV product's (no
-// transposing MFMAs): source lane s of group g addresses V row 4g + s / 4
-// (+ 16), columns 16 db + 4 (s % 4) .. + 3, and lane (d, g) gets keys 4g + i.
+// operand. bf16 takes V through ds_read_b64_tr_b16 straight into the PV
+// product's A (no transposing MFMAs): source lane s of group g addresses V row
+// 4g + s / 4 (+ 16), columns 16 db + 4 (s % 4) .. + 3, and lane (d, g) gets
+// keys 4g + i; the weights go in as three bf16 parts, exactly. fp16 parts
+// cannot hold a float32 weight (their least value is 2^-24), so fp16 takes the
+// PV product of float32 below, lane (r, g) reading V[tok 4g + i][4r .. +3] (8
+// bytes; 16 lanes a whole row) from the staging and widening it.
 //
 // float32: 16-token steps on v_mfma_f32_16x16x4_f32 (A[r][g], B[g][r],
 // C[4g+i][r]), every product and sum float32. K through the staging (chunk c
@@ -809,8 +813,9 @@ void attn_decode_stream(
 // float32 32 / 8 heads, D = 128, one row of 16384 tokens 109 -> 32 us (4.1
 // TB/s); 16 rows of 100-8000 tokens, paged, 447 -> 117 us (4.6 TB/s); bf16,
 // D = 64, 64 such rows 1050 -> 110 us (4.7 TB/s); 4 rows of 128-1024 tokens,
-// bf16, D = 64, 26.8 -> 12.3 us (graph replays). Error against 64 bits, f32:
-// 2.0e-7 where the general kernel has 2.7e-7 (16384 tokens).
+// bf16, D = 64, 26.8 -> 12.3 us (graph replays); fp16, D = 64, pays ~10% for
+// its float32 PV (64 rows of 100-8000 tokens 116 us, bf16 104). Error against
+// 64 bits, f32: 2.0e-7 where the general kernel has 2.7e-7 (16384 tokens).
 // ---------------------------------------------------------------------------
 template <typename T, int D>
 struct WideStep {
@@ -843,6 +848,7 @@ void attn_decode_wide(
     int min_seg, int low_seg, int cus) {
     using W = WideStep<T, D>;
     constexpr bool F32 = W::kF32;
+    constexpr bool PV32 = !std::is_same<T, bf16>::value;  // PV on the float32 MFMA
     constexpr bool PAGED = MODE != kRowsContig;
     constexpr int kTok = W::kTok, kRows = W::kRows, kRowLanes = W::kRowLanes;
     constexpr int kElems = 16 / (int)sizeof(T);  // elements per 16-byte chunk
@@ -1021,7 +1027,7 @@ void attn_decode_wide(
                     psum += s[h][i];
                 }
             l_run = l_run * alpha + psum;
-            if constexpr (F32) {
+            if constexpr (PV32) {
                 // the step's own sum first: one rounding a step in acc
 #pragma unroll
                 for (int hh = 0; hh < D / 64; ++hh) {
@@ -1029,12 +1035,22 @@ void attn_decode_wide(
 #pragma unroll
                     for (int c = 0; c < 4; ++c) sum[c] = odd[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const f32x4 vv = __builtin_bit_cast(f32x4, vin[i * (D / 64) + hh]);
+                    for (int x = 0; x < 4 * W::kTiles; ++x) {  // token 16h + 4g + i
+                        const int h = x >> 2, i = x & 3;
+                        float vv[4];
+                        if constexpr (F32) {
+                            const f32x4 v4 = __builtin_bit_cast(f32x4, vin[i * (D / 64) + hh]);
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) vv[c] = v4[c];
+                        } else {
+                            const float4 v4 = St<T>::ld4(reinterpret_cast<const T*>(
+                                stg + W::kStage + at(16 * h + 4 * g + i, r >> 1) + 8 * (r & 1)));
+                            vv[0] = v4.x, vv[1] = v4.y, vv[2] = v4.z, vv[3] = v4.w;
+                        }
 #pragma unroll
                         for (int c = 0; c < 4; ++c) {
-                            f32x4& x = i & 1 ? odd[c] : sum[c];
-                            x = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[c], s[0][i], x, 0, 0, 0);
+                            f32x4& y = i & 1 ? odd[c] : sum[c];
+                            y = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[c], s[h][i], y, 0, 0, 0);
                         }
                     }
 #pragma unroll
@@ -1051,28 +1067,21 @@ void attn_decode_wide(
                 using V8 = typename Mfma<T>::v8;
                 typedef short v4s __attribute__((ext_vector_type(4)));
                 typedef short v8s __attribute__((ext_vector_type(8)));
-                // the weights in parts of T, truncated: all 24 significant
-                // bits (3 bf16) or 22 (2 fp16). No part is 0 unless the weight
-                // is, so every product of a weight and an infinite V value is
-                // that infinity (the general kernel's result)
-                constexpr int kParts = std::is_same<T, bf16>::value ? 3 : 2;
-                V8 pp[kParts];
+                // the weights in three bf16 parts, truncated: all 24 significant
+                // bits. No part is 0 unless the weight is (exp2f here has no
+                // subnormal results, so its first part is not), so every
+                // product of a weight and an infinite V value is that infinity
+                // (the general kernel's result)
+                V8 pp[3];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const float p = s[i >> 2][i & 3];
                     float rest = p;
 #pragma unroll
-                    for (int x = 0; x < kParts; ++x) {
-                        float hi, least;
-                        if constexpr (std::is_same<T, bf16>::value) {
-                            hi = __uint_as_float(__float_as_uint(rest) & 0xffff0000u);
-                            least = 0x1p-126f;
-                        } else {
-                            hi = (float)__builtin_amdgcn_cvt_pkrtz(rest, 0.f)[0];
-                            least = 0x1p-24f;
-                        }
+                    for (int x = 0; x < 3; ++x) {
+                        const float hi = __uint_as_float(__float_as_uint(rest) & 0xffff0000u);
                         rest -= hi;
-                        pp[x][i] = (T)(x > 0 && p > 0.f ? fmaxf(hi, least) : hi);
+                        pp[x][i] = (T)(x > 0 && p > 0.f ? fmaxf(hi, 0x1p-126f) : hi);
                     }
                 }
 #pragma unroll
@@ -1088,7 +1097,7 @@ void attn_decode_wide(
                     const V8 va = __builtin_bit_cast(
                         V8, v8s{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
 #pragma unroll
-                    for (int x = 0; x < kParts; ++x)
+                    for (int x = 0; x < 3; ++x)
                         acc[db] = Mfma<T>::mma(va, pp[x], acc[db]);
                 }
             }
@@ -1130,8 +1139,8 @@ void attn_decode_wide(
         for (int nn = 0; nn < D / 16; ++nn)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                // acc[4h + c][i] of float32: dim 64h + 16g + 4i + c
-                const int d = F32 ? 64 * (nn >> 2) + 16 * g + 4 * i + (nn & 3)
+                // acc[4h + c][i] of the float32 PV: dim 64h + 16g + 4i + c
+                const int d = PV32 ? 64 * (nn >> 2) + 16 * g + 4 * i + (nn & 3)
                                   : 16 * nn + 4 * g + i;
                 s_acc[wave][r][d] = acc[nn][i];
             }

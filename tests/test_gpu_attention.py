@@ -673,3 +673,70 @@ def test_append_decode_of_64_dims(dt):
         torch.cuda.synchronize()
         assert torch.equal(again, out)
         ft.attention_decode_paged(args[0], k1, v1, args[3], args[6])  # eager work between
+
+
+def _decode_f64(q, k, v, lens):
+    """Contiguous decode in 64 bits; -inf and NaN as the formula gives them,
+    except that a weight below float32's least normal is 0 and drops its V."""
+    b, hq, d = q.shape
+    out = np.zeros((b, hq, d))
+    for i in range(b):
+        for h in range(hq):
+            n, kv = lens[i], h // (hq // k.shape[1])
+            s = (k[i, kv, :n].astype(np.float64) @ q[i, h]) / np.sqrt(d)
+            w = np.exp(s - s.max())
+            vv = v[i, kv, :n].astype(np.float64)
+            out[i, h] = w[w > 0] @ vv[w > 0] / w.sum()
+    return out
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("segs", [0, 1])
+def test_wide_decode_small_weights_count_as_much_as_they_weigh(dt, segs, tuning):
+    # four keys (one in each wave's first step) far above the 8188 others,
+    # with V = 0 there and V = vbig elsewhere: the output is the sum of the
+    # small weights, 17 to 32 nats below the dominant ones. Scores are exact
+    # products of one dim (q0 * k0, at most 2^9), so the weights are off by
+    # float32's rounding of the exponent (|s| log2(e) 2^-24 < 2^-14 with a
+    # margin of two) and the output by the storage rounding: 2^-p for p
+    # significant bits (fp16 11, bf16 8), fp16's subnormals half of 2^-24.
+    # One segment keeps all of a row's keys in one online softmax.
+    d, n, hkv, group = 64, 8192, 2, 4
+    q = np.zeros((1, hkv * group, d), np.float32)
+    k = np.zeros((1, hkv, n, d), np.float32)
+    gaps = np.array([17, 20, 25, 32], np.float32)
+    q[0, :, 0] = np.tile(8 * gaps / 16, hkv)   # s = k0 * gap / 16
+    k[0, :, (0, 32, 64, 96), 0] = 16.0
+    vbig = np.array([1.0, 3e4], np.float32)[:, None, None]
+    v = np.broadcast_to(vbig, (hkv, n, d)).copy()[None]
+    v[0, :, (0, 32, 64, 96)] = 0.0
+    lens = np.array([n], np.int32)
+    if segs:
+        tuning("FT_ATTN_SEGS", segs)
+    got = ft.attention_decode(t(q, dt), t(k, dt), t(v, dt), t(lens)).double().cpu().numpy()
+    ref = _decode_f64(rounded(q, dt), rounded(k, dt), rounded(v, dt), lens)
+    assert (ref > 0).all()
+    half_ulp, least = (2.0 ** -11, 2.0 ** -25) if dt is torch.float16 else (2.0 ** -8, 0.0)
+    np.testing.assert_allclose(got, ref, rtol=half_ulp + 2.0 ** -13, atol=least)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_wide_decode_infinite_value_at_a_small_weight(dt, tuning):
+    # 25 nats (2^-36) below the row's maximum an infinite V is still that
+    # infinity in its column, as on the general kernel, and no other column's
+    d, n = 64, 300
+    q = np.zeros((1, 2, d), np.float32)
+    k = np.zeros((1, 2, n, d), np.float32)
+    v = np.ones((1, 2, n, d), np.float32)
+    q[0, :, 0] = 8.0
+    k[0, :, 7, 0] = 25.0
+    v[0, :, 9, 3] = np.inf     # the dominant key's step
+    v[0, :, 200, 11] = -np.inf  # another step
+    args = (t(q, dt), t(k, dt), t(v, dt), t(np.array([n], np.int32)))
+    tuning("FT_ATTN_SEGS", 1)
+    got = ft.attention_decode(*args).float().cpu().numpy()
+    tuning("FT_ATTN_FORCE_GENERIC", 1)
+    ref = ft.attention_decode(*args).float().cpu().numpy()
+    assert np.isposinf(ref[..., 3]).all() and np.isneginf(ref[..., 11]).all()
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+    np.testing.assert_allclose(got, ref, rtol=2.0 ** -8)
