@@ -1546,8 +1546,8 @@ struct Workspace {
         if (!fixed) {
             try {
                 return scratch(Scratch::AttnPartials, bytes, s);
-            } catch (const Error& err) {
-                if (!fallback || err.code != FT_EHIP || bytes > FT_NOALLOC_WORKSPACE_BYTES) throw;
+            } catch (const NoRoom&) {
+                if (!fallback || bytes > FT_NOALLOC_WORKSPACE_BYTES) throw;
                 return fallback();
             }
         }
@@ -1686,10 +1686,10 @@ int attention_run(const T* q, const T* k, const T* v, const int* table,
             char* ws = nullptr;
             try {
                 ws = (char*)wsp.get(bytes, s);
-            } catch (const Error& err) {
-                // no room (or a capture before the shape's first call): the
-                // general kernel may need less
-                if (err.code != FT_EHIP || half128 || ap.k_new) throw;
+            } catch (const NoRoom&) {
+                // (or a capture before the shape's first call): the general
+                // kernel may need less
+                if (half128 || ap.k_new) throw;
             }
             if (ws && dim == kMfmaDim)
                 return attention_stream_run<T, 128>(
@@ -1833,8 +1833,8 @@ void attention_append_run(const T* q, T* k_pool, T* v_pool, const int* table, co
             attention_run<T>(q, k_pool, v_pool, table, lens, out, batch, hq, hkv, page, tbl_width,
                              dim, true, s, Workspace{}, nullptr, nullptr, nullptr, ap);
             return;
-        } catch (const Error& err) {  // no workspace: the two ops may need less
-            if (err.code != FT_EHIP || dim == kMfmaDim) throw;
+        } catch (const NoRoom&) {  // no workspace: the two ops may need less
+            if (dim == kMfmaDim) throw;
         }
     }
     kv_append_run<T>(k_new, v_new, table, lens, k_pool, v_pool, batch, hkv, dim, page,

@@ -27,6 +27,12 @@ struct Error {
     std::string msg;
 };
 
+// Scratch that cannot be had (no device memory, or growth under a capture),
+// nothing launched: a caller with a path that needs less may take it. Every
+// other HIP failure - a launch, or an earlier kernel's fault that shows in the
+// next call - is a plain Error, which no caller may answer with another path.
+struct NoRoom : Error {};
+
 [[noreturn]] inline void inval(const std::string& msg) {
     throw Error{FT_EINVAL, msg};
 }
@@ -109,8 +115,8 @@ enum class Tune : int {
     ArgSlices,             // FT_ARG_SLICES: argmax_batched slices per row
     SmpSingle,             // FT_SMP_SINGLE: sampling, one workgroup per row
     SmpSlices,             // FT_SMP_SLICES: sampling slices per row
-    FailScratch,           // FT_FAIL_SCRATCH (test hook): every scratch request
-                           // fails as an allocation failure would
+    FailScratch,           // FT_FAIL_SCRATCH (test hook): 1 every scratch request
+                           // fails for want of memory, 2 with another HIP error
     PrefillPrepass,        // FT_PREFILL_PREPASS: bf16 V to fp16 in a pre-pass
                            // (0 never: in the kernel; 1 large calls; 2 always)
     GridSync,              // FT_GRID_SYNC: bit mask of the per-tensor maxima not

@@ -523,8 +523,7 @@ bool grid_room(int nwg, hipStream_t s, GridMax& gm) {
     try {
         gm = gridmax_state(nwg, s);
         return true;
-    } catch (const Error& err) {
-        if (err.code != FT_EHIP) throw;
+    } catch (const NoRoom&) {
         return false;
     }
 }
@@ -547,8 +546,8 @@ void rmsq_rows_run(const T* x, const RmsqIo<T>& io, const float* w, const T* r,
     if (!can_grid || rows > kRmsqGridRows) {
         try {
             stat = (RowStat*)scratch(Scratch::QuantMax, (size_t)rows * sizeof(RowStat), s);
-        } catch (const Error& err) {
-            if (err.code != FT_EHIP || !can_grid) throw;
+        } catch (const NoRoom&) {
+            if (!can_grid) throw;
         }
     }
     GridMax gm{};

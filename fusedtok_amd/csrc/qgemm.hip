@@ -2324,9 +2324,9 @@ bool qgemm_mid_dispatch(const i8* a, const i8* b, const Epi& e, int m, int n, in
         try {
             part = (int*)scratch(Scratch::GemmPartials,
                                  (size_t)pick.ksplit * m * n * sizeof(int), s);
-        } catch (const Error& err) {
-            // no room for partials (or a capture before the first call): unsplit
-            if (err.code != FT_EHIP || forced > 0) throw;
+        } catch (const NoRoom&) {
+            // (or a capture before the first call): unsplit
+            if (forced > 0) throw;
             pick = mid_pick(m, n, k, cus, false);
             if (big && big_us(m, n, k, cus) <= pick.us) return false;
         }

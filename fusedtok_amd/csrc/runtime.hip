@@ -131,17 +131,21 @@ constexpr int kGridMostWgs = 4096;  // workgroups per state
 void* scratch_impl(Scratch which, size_t bytes, hipStream_t s, bool zero) {
     // test hook, checked before any HIP call so that a host without a
     // device reaches it too
-    if (tune(Tune::FailScratch, 0))
-        throw Error{FT_EHIP, "device scratch allocation: out of memory "
+    const int fail = tune(Tune::FailScratch, 0);
+    if (fail == 2)
+        throw Error{FT_EHIP, "device scratch allocation: a HIP error "
                              "(simulated by FT_FAIL_SCRATCH)"};
+    if (fail)
+        throw NoRoom{{FT_EHIP, "device scratch allocation: out of memory "
+                               "(simulated by FT_FAIL_SCRATCH)"}};
     const int dev = current_device();
     std::lock_guard<std::mutex> lock(state_mutex());
     ScratchSlot& slot = state_for(dev).slots[(int)which];
     if (slot.bytes >= bytes && slot.ptr) return slot.ptr;
     if (stream_capturing(s))
-        throw Error{FT_EHIP,
-                    "device scratch must grow outside a HIP graph capture: "
-                    "run the shape once before capturing it"};
+        throw NoRoom{{FT_EHIP,
+                      "device scratch must grow outside a HIP graph capture: "
+                      "run the shape once before capturing it"}};
     // A grown slot's old buffer is retired, never freed: in-flight kernels
     // and HIP graphs captured earlier still hold its address. Growth is
     // geometric, so a process retires at most a few dozen buffers.
@@ -152,6 +156,11 @@ void* scratch_impl(Scratch which, size_t bytes, hipStream_t s, bool zero) {
     hipError_t e = hipMalloc(&p, want);
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        // (an allocation another stream's capture forbids counts as no room)
+        if (e == hipErrorOutOfMemory ||
+            (e >= hipErrorStreamCaptureUnsupported && e <= hipErrorStreamCaptureWrongThread))
+            throw NoRoom{{FT_EHIP, std::string("device scratch allocation: ") +
+                                       hipGetErrorString(e)}};
         hip_fail("device scratch allocation", e);
     }
     if (zero) {

@@ -1047,8 +1047,7 @@ void topp_launch(const float* x, int rows, int n, float p, float t, float pen,
     char* ws = nullptr;
     try {
         ws = (char*)scratch(Scratch::Sampling, off, s);
-    } catch (const Error& err) {  // no room (or a capture before the first call)
-        if (err.code != FT_EHIP) throw;
+    } catch (const NoRoom&) {  // (or a capture before the first call)
         return one_workgroup_per_row();
     }
     a.bits = (unsigned*)(ws + o_bits);

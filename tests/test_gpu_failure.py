@@ -81,3 +81,40 @@ def test_quantize_raises_above_one_launch_and_runs_below(tuning):
     tuning.clear("FT_FAIL_SCRATCH")
     _, s2 = ft.quantize_int8(big)
     assert s2 == float(np.float32(big.abs().max().item()) / np.float32(127.0))
+
+
+def test_an_error_that_is_not_want_of_memory_is_reported(tuning):
+    # FT_FAIL_SCRATCH=2: the scratch request fails with another HIP error (an
+    # earlier kernel's fault shows so). The steps that answer want of memory
+    # with another path must raise it, each of them.
+    x = torch.randn(8, 4096, device=DEV)
+    x100 = torch.randn(100, 4096, device=DEV)
+    w = torch.ones(4096, device=DEV)
+    rng = np.random.default_rng(5)
+    q, kp, vp, tbl, ln = (t(a) for a in paged(rng, d=64))
+    kn = torch.randn(3, 4, 64, device=DEV)
+    a = torch.ones(150, 4096, dtype=torch.int8, device=DEV)
+    b = torch.ones(1024, 4096, dtype=torch.int8, device=DEV)
+    sb = torch.ones(1024, device=DEV)
+    half = [y.half() for y in (q, kp, vp)]
+    calls = dict(
+        rmsnorm_one_launch=lambda: ft.rmsnorm_quant(x, w),
+        rmsnorm_two_launches=lambda: ft.rmsnorm_quant(x100, w),
+        swiglu=lambda: ft.swiglu_quant(x, x),
+        sampling=lambda: ft.sample_topp_batched(torch.randn(2, 32768, device=DEV), 0.9,
+                                                seeds=[1, 2]),
+        gemm=lambda: ft.qgemm_perchannel(a, 0.1, b, sb),
+        decode=lambda: ft.attention_decode_paged(q, kp, vp, tbl, ln),
+        contiguous=lambda: ft.attention_decode(q, kp.view(-1, 4, 16, 64)[:3].contiguous(),
+                                               vp.view(-1, 4, 16, 64)[:3].contiguous(),
+                                               torch.full_like(ln, 9)),
+        append=lambda: ft.attention_decode_paged_append(half[0], half[1], half[2], tbl,
+                                                        kn.half(), kn.half(), ln))
+    for name, call in calls.items():
+        call()
+        tuning("FT_FAIL_SCRATCH", 2)
+        with pytest.raises(RuntimeError, match="a HIP error"):
+            call()
+            pytest.fail(f"{name} took another path")
+        tuning.clear("FT_FAIL_SCRATCH")
+        call()
