@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -1576,11 +1577,20 @@ int attention_stream_run(const T* q, const T* k, const T* v, const int* table, c
     float* ws_acc = ws_ml + ((nslots * 2 + 63) & ~(size_t)63);
     long long* pref = (long long*)(ws_acc + nslots * D);
     if (ap.k_new && (amax || qcodes)) inval("attention: the append form keeps no per-head maxima");
+    const long long heads = (long long)batch * hq;
+    // the quantizing combine's state, had before anything is launched
+    const long long cq_wgs = (heads + kCqWaves - 1) / kCqWaves;
+    GridMax gm{};
+    bool one_combine = false;
+    if (qcodes && cq_wgs <= (1 << 16)) {
+        gm = gridmax_state((int)cq_wgs, s);
+        one_combine = grid_resident((const void*)attn_combine_quant<T, D>, (int)cq_wgs,
+                                    64 * kCqWaves, GridUse::AttnOut);
+    }
     launch_stream<T, D>(paged, page_shift, nseg, s, q, k, v, table, lens, ws_ml, ws_acc, pref,
                         out, batch, hq, hkv, group, rows_or_page, tbl_width, span, scale_log2,
                         min_seg, low_seg, ap.k_new != nullptr, cus);
     launch_check("attention decode kernel launch");
-    const long long heads = (long long)batch * hq;
     if (ap.k_new) {
         if (page_shift >= 0)
             attn_combine_append<T, D, kRowsPagedPow2><<<(unsigned)heads, 64, 0, s>>>(
@@ -1593,18 +1603,11 @@ int attention_stream_run(const T* q, const T* k, const T* v, const int* table, c
         launch_check("attention combine + append kernel launch");
         return 0;
     }
-    if (qcodes) {
-        const long long nwg = (heads + kCqWaves - 1) / kCqWaves;
-        if (nwg <= (1 << 16)) {
-            const GridMax gm = gridmax_state((int)nwg, s);
-            if (grid_resident((const void*)attn_combine_quant<T, D>, (int)nwg, 64 * kCqWaves,
-                              GridUse::AttnOut)) {
-                attn_combine_quant<T, D><<<(unsigned)nwg, 64 * kCqWaves, 0, s>>>(
-                    ws_ml, ws_acc, pref, out, qcodes, qscale, batch, hq, hkv, group, gm);
-                launch_check("attention combine + quantize kernel launch");
-                return 2;
-            }
-        }
+    if (one_combine) {
+        attn_combine_quant<T, D><<<(unsigned)cq_wgs, 64 * kCqWaves, 0, s>>>(
+            ws_ml, ws_acc, pref, out, qcodes, qscale, batch, hq, hkv, group, gm);
+        launch_check("attention combine + quantize kernel launch");
+        return 2;
     }
     if (amax)
         attn_combine_stream<T, D, true><<<(unsigned)heads, 64, 0, s>>>(
@@ -1616,14 +1619,16 @@ int attention_stream_run(const T* q, const T* k, const T* v, const int* table, c
     return amax ? 1 : 0;
 }
 
-// As attention_stream_run, whatever the shape.
+// As attention_stream_run, whatever the shape. `first` (where given) launches
+// what comes before the decode, once the decode's memory is had.
 template <typename T>
 int attention_run(const T* q, const T* k, const T* v, const int* table,
                    const int* lens, T* out, int batch, int hq, int hkv,
                    int rows_or_page, int tbl_width, int dim, bool paged,
                    hipStream_t s, const Workspace& wsp = Workspace{},
                    float* amax = nullptr, signed char* qcodes = nullptr,
-                   float* qscale = nullptr, const AppendArgs<T>& ap = AppendArgs<T>{}) {
+                   float* qscale = nullptr, const AppendArgs<T>& ap = AppendArgs<T>{},
+                   const std::function<void()>& first = nullptr) {
     long long span;
     if (paged) {
         span = (long long)tbl_width * rows_or_page;
@@ -1691,6 +1696,7 @@ int attention_run(const T* q, const T* k, const T* v, const int* table,
                 // kernel may need less
                 if (half128 || ap.k_new) throw;
             }
+            if (ws && first) first();
             if (ws && dim == kMfmaDim)
                 return attention_stream_run<T, 128>(
                     q, k, v, table, lens, out, batch, hq, hkv, rows_or_page, page_shift,
@@ -1707,6 +1713,7 @@ int attention_run(const T* q, const T* k, const T* v, const int* table,
     if (units * 256 > (1LL << 31)) inval("attention problem too large for one launch");
     float* ws_ml = (float*)wsp.get(gen_bytes, s);
     float* ws_acc = ws_ml + (((size_t)units * group * 2 + 63) & ~(size_t)63);
+    if (first) first();
     RowMap rm;
     rm.table = paged ? table : nullptr;
     rm.hkv = hkv;
@@ -1764,7 +1771,7 @@ template <typename T>
 void kv_append_run(const T* k_new, const T* v_new, const int* table,
                    const int* lens, T* k_dst, T* v_dst, int batch, int hkv,
                    int dim, int rows_or_page, int tbl_width, bool paged,
-                   hipStream_t s) {
+                   hipStream_t s, bool check_only = false) {
     if (batch <= 0) return;  // nothing to append (reference attention.cu:1930-1931)
     if (dim % 4 != 0) inval("dim must be a multiple of 4");
     if (paged && rows_or_page < 1) inval("page size must be >= 1");
@@ -1791,6 +1798,7 @@ void kv_append_run(const T* k_new, const T* v_new, const int* table,
     const int chunks = hkv * (dim / 4);
     const int per_row = (chunks + 255) / 256;
     if ((long long)batch * per_row > (1LL << 31) - 1) inval("kv append: batch too large");
+    if (check_only) return;
     kv_append_kernel<T><<<(unsigned)(batch * per_row), 256, 0, s>>>(
         k_new, v_new, lens, rm, (int)cap, per_row, k_dst, v_dst);
     launch_check("kv append kernel launch");
@@ -1808,7 +1816,9 @@ __global__ __launch_bounds__(256) void lens_plus1_kernel(const int* __restrict__
 // kernel attends the lens[b] cached tokens (every piece leaves a partial)
 // and attn_combine_append folds the fresh token from k_new / v_new into
 // each row's log-sum-exp merge (float32) and writes it to the pools - one
-// launch fewer. Elsewhere: the two ops, lens + 1 through library scratch.
+// launch fewer. Elsewhere: the two ops, lens + 1 through library scratch, the
+// append enqueued once the decode's memory is had: a call that fails for want
+// of memory leaves the pools as they were.
 template <typename T>
 void attention_append_run(const T* q, T* k_pool, T* v_pool, const int* table, const T* k_new,
                           const T* v_new, const int* lens, T* out, int batch, int hq, int hkv,
@@ -1837,13 +1847,19 @@ void attention_append_run(const T* q, T* k_pool, T* v_pool, const int* table, co
             if (dim == kMfmaDim) throw;
         }
     }
-    kv_append_run<T>(k_new, v_new, table, lens, k_pool, v_pool, batch, hkv, dim, page,
-                     tbl_width, true, s);
+    auto append = [&](bool check_only) {
+        kv_append_run<T>(k_new, v_new, table, lens, k_pool, v_pool, batch, hkv, dim, page,
+                         tbl_width, true, s, check_only);
+    };
+    append(true);
     int* lens1 = (int*)scratch(Scratch::AttnLens, (size_t)batch * sizeof(int), s);
-    lens_plus1_kernel<<<(unsigned)((batch + 255) / 256), 256, 0, s>>>(lens, lens1, batch);
-    launch_check("lens + 1 kernel launch");
     attention_run<T>(q, k_pool, v_pool, table, lens1, out, batch, hq, hkv, page, tbl_width, dim,
-                     true, s);
+                     true, s, Workspace{}, nullptr, nullptr, nullptr, AppendArgs<T>{}, [&] {
+                         append(false);
+                         lens_plus1_kernel<<<(unsigned)((batch + 255) / 256), 256, 0, s>>>(
+                             lens, lens1, batch);
+                         launch_check("lens + 1 kernel launch");
+                     });
 }
 
 }  // namespace

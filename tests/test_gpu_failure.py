@@ -118,3 +118,32 @@ def test_an_error_that_is_not_want_of_memory_is_reported(tuning):
             pytest.fail(f"{name} took another path")
         tuning.clear("FT_FAIL_SCRATCH")
         call()
+
+
+@pytest.mark.parametrize("dt,d", [(torch.float32, 128), (torch.float16, 64), (torch.bfloat16, 128),
+                                  (torch.bfloat16, 48)])
+@pytest.mark.parametrize("fail", [1, 16 << 0, 16 << 6])
+def test_append_decode_without_memory_leaves_the_pools(dt, d, fail, tuning):
+    # every request fails; the decode's partials alone; lens + 1 alone (which
+    # the one-call form does not need)
+    rng = np.random.default_rng(6)
+    q, kp, vp, tbl, ln = paged(rng, d=d)
+    k1, v1 = t(kp, dt), t(vp, dt)
+    kn, vn = (torch.randn(3, 4, d, device=DEV).to(dt) for _ in range(2))
+    args = (t(q, dt), k1, v1, t(tbl), kn, vn, t(ln))
+    k0, v0 = k1.clone(), v1.clone()
+    one_call = dt is not torch.float32 and d in (64, 128)
+    tuning("FT_FAIL_SCRATCH", fail)
+    if fail == 16 << 6 and one_call:
+        ft.attention_decode_paged_append(*args)
+    else:
+        with pytest.raises(RuntimeError, match="out of memory"):
+            ft.attention_decode_paged_append(*args)
+        assert torch.equal(k1, k0) and torch.equal(v1, v0)
+    tuning.clear("FT_FAIL_SCRATCH")
+    got = ft.attention_decode_paged_append(*args)
+    ft.kv_append_paged(k0, v0, args[3], kn, vn, args[6])
+    assert torch.equal(k1, k0) and torch.equal(v1, v0)
+    ref = oracle.attention_decode_paged(args[0].float().cpu().numpy(), k0.float().cpu().numpy(),
+                                        v0.float().cpu().numpy(), tbl, ln + 1)
+    np.testing.assert_allclose(got.float().cpu().numpy(), ref, rtol=1e-2, atol=2e-3)
