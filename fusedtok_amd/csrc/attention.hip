@@ -323,11 +323,12 @@ constexpr int kStreamScanRows = 2048;        // sequences per launch (LDS prefix
 // 20.0 us at 512, 21.3 us at 256.
 constexpr int kStreamMinSeg = 512;
 // A call too small to give every CU that many takes shorter segments, one
-// per CU, down to this (bf16, 4 rows of 10-2000 tokens, 8 kv heads: 16.4 us
-// against 23.3 with 512 tokens) - or to half of it where those still leave
-// CUs idle (fp16, D = 64, 4 rows of 10-200 tokens: 14.3 against 17.5 us; four
-// rows of 128-1024 tokens, which do not, are better off at 128: 11.7 against
-// 12.7 us with 64).
+// per CU, down to this (bf16, 4 rows of 10-2000 tokens, 8 kv heads: 13.6 us
+// against 22.5 with 512 tokens) - or to half of it where those still leave
+// CUs idle (D = 64, 4 rows of 10-200 tokens, 2.3k flat tokens: bf16 14.2
+// against 18.1 us, fp16 15.9 against 20.7). The line is where 64-token
+// segments fill the CUs; near it 128 is the better (13.5k flat tokens, bf16,
+// D = 64: 10.9 against 11.6 us).
 constexpr int kStreamLowSeg = 128;
 
 // Rows of equal length, each at least this long, take one segment per CU
@@ -395,11 +396,12 @@ __device__ __forceinline__ long long uniform64(long long x) {
 // or, when that would leave CUs without a segment (cus > 0: their count), as
 // many as give each CU one, down to low_seg (half of it where even those
 // leave CUs without one: short rows, where a segment holds several pieces).
+// low_seg 0: min_seg whatever the CUs (FT_ATTN_MIN_SEG).
 __device__ __forceinline__ long long stream_seg_len(long long total, int nseg, int min_seg,
                                                     int low_seg, int cus) {
     const long long s = (total + nseg - 1) / nseg;
     long long least = min_seg;
-    if (cus > 0) {
+    if (cus > 0 && low_seg > 0) {
         const long long low = total <= (long long)cus * (low_seg / 2) ? low_seg / 2 : low_seg;
         least = max(low, min(least, (total + cus - 1) / cus));
     }
@@ -1682,7 +1684,7 @@ int attention_run(const T* q, const T* k, const T* v, const int* table,
         const int cus = forced > 0 ? 0 : cu_count;
         const int tuned_seg = tune(Tune::AttnMinSeg, 0);
         const int min_seg = std::max(32, tuned_seg > 0 ? tuned_seg : kStreamMinSeg);
-        const int low_seg = tuned_seg > 0 ? min_seg : kStreamLowSeg;
+        const int low_seg = tuned_seg > 0 ? 0 : kStreamLowSeg;
         const size_t bytes = ws_bytes(((size_t)nseg + (size_t)batch * hkv) * group) +
                              (batch + 2) * sizeof(long long);
         // a bounded workspace that only the general kernel's partials fit

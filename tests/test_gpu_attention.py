@@ -740,3 +740,27 @@ def test_wide_decode_infinite_value_at_a_small_weight(dt, tuning):
     assert np.isposinf(ref[..., 3]).all() and np.isneginf(ref[..., 11]).all()
     np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
     np.testing.assert_allclose(got, ref, rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("dt,d", WIDE + [(torch.bfloat16, 128)])
+def test_min_seg_is_a_minimum_for_small_calls_too(dt, d, tuning):
+    # 2964 flat tokens: FT_ATTN_MIN_SEG=32 gives the 93 segments of 32 tokens
+    # that FT_ATTN_SEGS asks for, bit for bit, and not shorter ones. Segments
+    # of 64 (what such a call takes unset) cut the rows elsewhere.
+    rng = np.random.default_rng(d)
+    q, k, v, _ = make_case(rng, 3, 16, 4, 705, d, False)
+    args = (t(q, dt), t(k, dt), t(v, dt), t(np.array([40, 700, 1], np.int32)))
+
+    def segments(min_seg, count=0):
+        tuning("FT_ATTN_MIN_SEG", min_seg)
+        if count:
+            tuning("FT_ATTN_SEGS", count)
+        out = ft.attention_decode(*args)
+        tuning.clear("FT_ATTN_SEGS")
+        tuning.clear("FT_ATTN_MIN_SEG")
+        return out
+
+    unset = ft.attention_decode(*args)
+    for n in (32, 64, 128):
+        assert torch.equal(segments(n), segments(n, (4 * 741 + n - 1) // n)), n
+    assert torch.equal(segments(64), unset) and not torch.equal(segments(32), unset)
