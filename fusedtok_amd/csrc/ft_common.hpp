@@ -15,6 +15,7 @@
 #include <string>
 
 #include "../../include/fusedtok_amd.h"
+#include "grid_word.hpp"
 
 namespace ft {
 
@@ -154,11 +155,13 @@ void* scratch_zeroed(Scratch which, size_t bytes, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Grid-wide maximum inside one launch (grid_max below). The state is one
-// 64-bit word (generation << 32 | arrivals) and one 32-bit slot per
-// workgroup, zeroed when allocated; every launch leaves the arrivals at 0.
-// Launches that use one state are ordered: a stream's launches share a state
-// and streams hash to 16 of them (calls that overlap on one GPU still race on
-// the library's other scratch).
+// 64-bit word (grid_word.hpp) and one 32-bit slot per workgroup, zeroed when
+// allocated; every launch leaves the arrivals at 0. Launches that use one
+// state must be ordered, which is the caller's duty as with the library's
+// other scratch: a stream's handle picks one of 16 states, so two streams can
+// share one, and a captured graph keeps its capture stream's on whatever
+// stream it is replayed. Launches that overlap on a state get wrong maxima,
+// later ones do not.
 struct GridMax {
     unsigned long long* word;
     unsigned* slots;
@@ -361,13 +364,25 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 // one coherence point, so no release fence (an L2 writeback per workgroup,
 // ~0.2 us each, serialised per XCD) is needed:
 //   1. exchange m into this workgroup's slot and wait until it is performed;
-//   2. arrive (add 1 to the word); the last arriver advances the generation
-//      and clears the arrivals with one add, the others poll the word until
-//      the generation moves (bounded: after kGridSpin polls, ~1 s, a
-//      workgroup goes on with the slots as they are, so a misuse gives wrong
-//      values and never a hang);
+//   2. arrive at the word (grid_arrive) and wait for the last arrival
+//      (bounded: after kGridSpin polls, ~1 s, a workgroup goes on with the
+//      slots as they are, so a misuse gives wrong values and never a hang);
 //   3. every slot now holds this launch's value: read them all.
 constexpr unsigned kGridSpin = 1u << 20;
+
+struct DeviceWord {
+    unsigned long long* p;
+    __device__ __forceinline__ grid_word_t add(grid_word_t x) const {
+        return __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void and_(grid_word_t x) const {
+        __hip_atomic_fetch_and(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ grid_word_t load() const {
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void pause() const { __builtin_amdgcn_s_sleep(8); }
+};
 
 template <int NT>
 __device__ __forceinline__ float grid_max(const GridMax& g, float m, float* red) {
@@ -378,20 +393,7 @@ __device__ __forceinline__ float grid_max(const GridMax& g, float m, float* red)
                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // the exchange has returned (so it was performed) before the arrival
         asm volatile("s_waitcnt vmcnt(0)" : : "v"(prev) : "memory");
-        const unsigned long long old = __hip_atomic_fetch_add(
-            g.word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned gen = (unsigned)(old >> 32);
-        if ((unsigned)old + 1u == nwg) {
-            __hip_atomic_fetch_add(g.word, (1ull << 32) - nwg, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            for (unsigned i = 0; i < kGridSpin; ++i) {
-                const unsigned long long cur =
-                    __hip_atomic_load(g.word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((unsigned)(cur >> 32) != gen) break;
-                __builtin_amdgcn_s_sleep(8);
-            }
-        }
+        grid_arrive(DeviceWord{g.word}, nwg, kGridSpin);
     }
     __syncthreads();
     float mx = 0.0f;

@@ -190,8 +190,7 @@ GridMax gridmax_state(int nwg, hipStream_t s) {
     // kGridStates states of one size, each a word and, from byte 256, the
     // slots; zeroed when allocated, and every launch leaves the arrivals at 0
     // (the generation keeps counting). A stream takes the state its handle
-    // hashes to: launches of one stream are ordered, and those of two streams
-    // that overlap then hardly ever meet on one counter.
+    // hashes to; streams that share a state must be ordered (GridMax).
     if (nwg > kGridMostWgs) nwg = kGridMostWgs;  // (more are never resident at once)
     constexpr size_t kState = 256 + 4 * (size_t)kGridMostWgs;
     char* p = (char*)scratch_zeroed(Scratch::GridSync, kGridStates * kState, s);
