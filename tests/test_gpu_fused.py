@@ -135,10 +135,13 @@ def test_rmsnorm_quant_one_launch_matches_two_launch_path(dt, rows, cols, tuning
 @pytest.mark.parametrize("rows,cols", [(17, 4096), (20, 12), (64, 4096), (64, 4),
                                        (257, 1028), (1000, 512), (4096, 64)])
 def test_rmsnorm_quant_grid_launch_matches_two_launches(dt, rows, cols, tuning):
-    # From 17 rows of at most 4096 columns, rmsnorm_quant is one launch: the
-    # tensor maximum is folded inside it through device-scope atomics
-    # (grid_max). FT_GRID_SYNC=1 forces the row pass + fold/quantize pair.
-    # Eight calls go back to back with no host sync, each with its largest
+    # Up to 64 rows of at most 4096 columns, and where there is no room for the
+    # row statistics up to as many as can be resident at once, rmsnorm_quant is
+    # one launch: the tensor maximum is folded inside it through device-scope
+    # atomics (grid_max). FT_FAIL_SCRATCH refuses the row statistics, so that
+    # the other row counts take it too (4096 rows are not resident: two
+    # launches both times). FT_GRID_SYNC=1 forces the row pass + fold/quantize
+    # pair. Eight calls go back to back with no host sync, each with its largest
     # value in another row, so a workgroup that read a stale maximum would
     # show as a wrong scale or wrong codes.
     rng = np.random.default_rng(rows * 17 + cols)
@@ -151,8 +154,11 @@ def test_rmsnorm_quant_grid_launch_matches_two_launches(dt, rows, cols, tuning):
         xs.append(t(a, dt))
         rs.append(t(rng.standard_normal((rows, cols)).astype(np.float32), dt))
     for with_res in (False, True):
+        if rows <= 1024:
+            tuning("FT_FAIL_SCRATCH", 16 << 1)  # Scratch::QuantMax
         got = [ft.rmsnorm_quant(x, w, residual=r if with_res else None, eps=1e-5,
                                 device_scale=True) for x, r in zip(xs, rs)]
+        tuning.clear("FT_FAIL_SCRATCH")
         tuning("FT_GRID_SYNC", 1)
         ref = [ft.rmsnorm_quant(x, w, residual=r if with_res else None, eps=1e-5,
                                 device_scale=True) for x, r in zip(xs, rs)]
@@ -162,8 +168,9 @@ def test_rmsnorm_quant_grid_launch_matches_two_launches(dt, rows, cols, tuning):
             assert torch.equal(q1, q2), f"call {i}: codes"
     # and against the oracle for the last call
     eq, es = oracle.rmsnorm_quant(as_f32(xs[-1]), w.cpu().numpy(), as_f32(rs[-1]), 1e-5)
-    np.testing.assert_array_equal(got[-1][0].cpu().numpy(), eq)
-    assert float(got[-1][1]) == es
+    for q, s in (got[-1], ref[-1]):
+        np.testing.assert_array_equal(q.cpu().numpy(), eq)
+        assert float(s) == es
 
 
 @pytest.mark.parametrize("dt", ALL)
@@ -700,7 +707,8 @@ def test_swiglu_quant_grid_launch_matches_two_launches(dt, rows, cols, tuning):
 @pytest.mark.parametrize("dt", ALL)
 @pytest.mark.parametrize("rows,cols", [(5, 4096), (6, 12), (16, 2048), (65, 1028)])
 def test_rmsnorm_quant_few_rows_match_two_launches(dt, rows, cols, tuning):
-    # one launch from 5 rows to 64, two from 65; the same codes either way
+    # one launch from 5 rows to 64, two from 65; the same codes either way, the
+    # oracle's
     rng = np.random.default_rng(rows + cols)
     w = t(rng.uniform(0.5, 1.5, cols).astype(np.float32))
     x, r = (t(rng.standard_normal((rows, cols)).astype(np.float32), dt) for _ in range(2))
@@ -710,3 +718,7 @@ def test_rmsnorm_quant_few_rows_match_two_launches(dt, rows, cols, tuning):
         q2, s2 = ft.rmsnorm_quant(x, w, residual=res, eps=1e-5)
         tuning.clear("FT_RMSQ_SPLIT")
         assert torch.equal(q1, q2) and s1 == s2
+        eq, es = oracle.rmsnorm_quant(as_f32(x), w.cpu().numpy(),
+                                      None if res is None else as_f32(res), 1e-5)
+        np.testing.assert_array_equal(q1.cpu().numpy(), eq)
+        assert s1 == es
