@@ -118,8 +118,9 @@ enum class Tune : int {
     SmpSlices,             // FT_SMP_SLICES: sampling slices per row
     FailScratch,           // FT_FAIL_SCRATCH (test hook): 1 every scratch request
                            // fails for want of memory, 2 with another HIP error;
-                           // from 16 those of the buffers b with bit 16 << b
-                           // set (Scratch), for want of memory
+                           // and for want of memory: from 16 those of the
+                           // buffers b with bit 16 << b set (Scratch), from
+                           // 4096 those of more bytes than the value
     PrefillPrepass,        // FT_PREFILL_PREPASS: bf16 V to fp16 in a pre-pass
                            // (0 never: in the kernel; 1 large calls; 2 always)
     GridSync,              // FT_GRID_SYNC: bit mask of the per-tensor maxima not

@@ -135,7 +135,8 @@ void* scratch_impl(Scratch which, size_t bytes, hipStream_t s, bool zero) {
     if (fail == 2)
         throw Error{FT_EHIP, "device scratch allocation: a HIP error "
                              "(simulated by FT_FAIL_SCRATCH)"};
-    if (fail == 1 || (fail >= 16 && (fail & (16 << (int)which))))
+    if (fail == 1 || (fail >= 4096 ? bytes > (size_t)fail
+                                   : fail >= 16 && (fail & (16 << (int)which))))
         throw NoRoom{{FT_EHIP, "device scratch allocation: out of memory "
                                "(simulated by FT_FAIL_SCRATCH)"}};
     const int dev = current_device();

@@ -147,3 +147,98 @@ def test_append_decode_without_memory_leaves_the_pools(dt, d, fail, tuning):
     ref = oracle.attention_decode_paged(args[0].float().cpu().numpy(), k0.float().cpu().numpy(),
                                         v0.float().cpu().numpy(), tbl, ln + 1)
     np.testing.assert_allclose(got.float().cpu().numpy(), ref, rtol=1e-2, atol=2e-3)
+
+
+# room for the general kernel's partials of the cases below (under 150 KB) but
+# not for the stream kernels' (256 or 512 segments more: over 270 KB)
+ROOM = 200 << 10
+
+
+@pytest.mark.parametrize("dt,d", [(torch.float32, 64), (torch.float32, 128), (torch.float16, 64),
+                                  (torch.bfloat16, 64)])
+def test_decode_with_room_for_the_general_kernel_alone(dt, d, tuning):
+    # the stream kernels' workspace cannot be had, in an eager call or under a
+    # capture: the general kernel's result bit for bit, and replays of it
+    rng = np.random.default_rng(7)
+    q, kp, vp, tbl, ln = paged(rng, hq=8, hkv=4, d=d, lens=(40, 400, 1))
+    args = (t(q, dt), t(kp, dt), t(vp, dt), t(tbl), t(ln))
+    stream = ft.attention_decode_paged(*args)
+    tuning("FT_ATTN_FORCE_GENERIC", 1)
+    want = ft.attention_decode_paged(*args)
+    tuning.clear("FT_ATTN_FORCE_GENERIC")
+    # so the two can be told apart (bf16's rounding can hide it)
+    assert dt is torch.bfloat16 or not torch.equal(stream, want)
+    tuning("FT_FAIL_SCRATCH", ROOM)
+    assert torch.equal(ft.attention_decode_paged(*args), want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ft.attention_decode_paged(*args)
+    tuning.clear("FT_FAIL_SCRATCH")
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        assert torch.equal(ft.attention_decode_paged(*args), stream)  # eager work between
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_append_decode_with_room_for_the_general_kernel_alone(dt, tuning):
+    # the appending form at D = 64 then is the append and the general decode
+    rng = np.random.default_rng(8)
+    q, kp, vp, tbl, ln = paged(rng, hq=8, hkv=4, d=64, lens=(40, 390, 1))
+    kn, vn = (torch.randn(3, 4, 64, device=DEV).to(dt) for _ in range(2))
+    qt, tt, lt = t(q, dt), t(tbl), t(ln)
+    k1, v1, k2, v2 = t(kp, dt), t(vp, dt), t(kp, dt), t(vp, dt)
+    ft.kv_append_paged(k2, v2, tt, kn, vn, lt)
+    tuning("FT_ATTN_FORCE_GENERIC", 1)
+    want = ft.attention_decode_paged(qt, k2, v2, tt, lt + 1)
+    tuning.clear("FT_ATTN_FORCE_GENERIC")
+    tuning("FT_FAIL_SCRATCH", ROOM)
+    got = ft.attention_decode_paged_append(qt, k1, v1, tt, kn, vn, lt)
+    assert torch.equal(got, want) and torch.equal(k1, k2) and torch.equal(v1, v2)
+    k3, v3 = t(kp, dt), t(vp, dt)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ft.attention_decode_paged_append(qt, k3, v3, tt, kn, vn, lt)
+    tuning.clear("FT_FAIL_SCRATCH")
+    for _ in range(3):
+        out.zero_()
+        k3.copy_(t(kp, dt))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(k3, k2) and torch.equal(v3, v2)
+
+
+def test_capture_without_warm_up_takes_the_paths_that_need_less(tuning):
+    # sampling and a K-split GEMM captured where their workspace cannot be had
+    # record one workgroup per row and no split: the same tokens and values
+    logits = torch.randn(3, 40000, device=DEV)
+    a = torch.randint(-127, 128, (150, 4096), dtype=torch.int8, device=DEV)
+    b = torch.randint(-127, 128, (1024, 4096), dtype=torch.int8, device=DEV)
+    sb = torch.rand(1024, device=DEV) * 0.01
+    sa = torch.full((1,), 0.02, device=DEV)
+    seeds = torch.tensor([1, 2, 3], device=DEV)
+
+    def sample():
+        out = torch.zeros(3, dtype=torch.int64, device=DEV)
+        ft._fusedtok.sample_topp_batched_launch(
+            logits.data_ptr(), 3, 40000, 0.9, 1.0, seeds.data_ptr(), out.data_ptr(),
+            torch.cuda.current_stream().cuda_stream)
+        return out
+
+    gemm = lambda: ft.qgemm_perchannel(a, sa, b, sb)  # noqa: E731
+    want_t, want_y = sample(), gemm()
+    assert want_t.tolist() == ft.sample_topp_batched(logits, 0.9, seeds=[1, 2, 3]).tolist()
+    tuning("FT_FAIL_SCRATCH", 1)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        toks, y = sample(), gemm()
+    tuning.clear("FT_FAIL_SCRATCH")
+    for _ in range(3):
+        toks.zero_()
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(toks, want_t) and torch.equal(y, want_y)
+        assert torch.equal(gemm(), want_y)  # eager work between

@@ -66,7 +66,7 @@ def run(lib, name, q, kp, vp, table, lens, out):
     # (seed, batch, q heads, kv heads, dim, lengths): the second call is smaller
     [(1, 24, 32, 8, 128, [4000, 1, 0, 17, 2048, 3333, 512, 4097] * 3),
      (2, 5, 16, 8, 128, [300, 77, 1, 1024, 33])],
-    # D = 64 takes the generic kernel, whose partials are laid out per chunk
+    # D = 64: partials half as wide
     [(3, 6, 8, 2, 64, [700, 0, 64, 1500, 5, 999]),
      (4, 2, 4, 4, 64, [129, 3])],
 ])
@@ -86,6 +86,21 @@ def test_noalloc_equals_the_allocating_entry_point(lib, case):
                                             vpt.float().cpu().numpy(), table, ln)
         err = np.abs(got.float().cpu().numpy() - ref) - (2e-3 + 1e-2 * np.abs(ref))
         assert err.max() <= 0, f"seed {seed}: outside 2e-3 + 1e-2|ref| of the oracle"
+
+
+def test_noalloc_of_64_dims_takes_the_general_kernel_where_only_that_fits(lib, tuning):
+    # 1900 rows x 2 kv heads x G 16: the stream's partials (512 segments more)
+    # are past the 16 MiB array, the general kernel's 60800 are not
+    q, kp, vp, table, ln = paged_case(5, 1900, 32, 2, 64, [32, 1, 17, 0, 31] * 380)
+    bf = torch.bfloat16
+    qt, kpt, vpt = (torch.from_numpy(a).to(DEV, bf) for a in (q, kp, vp))
+    tt, lt = torch.from_numpy(table).to(DEV), torch.from_numpy(ln).to(DEV)
+    want, got = (torch.full(qt.shape, float("nan"), dtype=bf, device=DEV) for _ in range(2))
+    run(lib, "ft_attention_decode_paged_launch_bf16_noalloc", qt, kpt, vpt, tt, lt, got)
+    tuning("FT_ATTN_FORCE_GENERIC", 1)
+    run(lib, "ft_attention_decode_paged_launch_bf16", qt, kpt, vpt, tt, lt, want)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
 
 
 def test_noalloc_rejects_a_call_beyond_the_static_workspace(lib):
