@@ -143,11 +143,18 @@ class Rule:
         self.exc = exc
 
 
+# torch's own raw calls, where this torch has them (they are not public)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def current_stream():
     """The current torch stream's handle on the current device, as an int
     (torch.cuda.current_stream().cuda_stream without building the Stream
-    object: 0.3 against 2 us)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    object: 0.3 against 2 us; by way of it where torch lacks the raw calls)."""
+    if _raw_stream is None or _raw_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 def _parse(shape):

@@ -231,3 +231,22 @@ def test_device_binding_equals_the_general_routines(contract, base, change):
 
     got = outcome(lambda values: contract.bind(**values))
     assert got == outcome(lambda values: _bind_by_the_general_routines(contract, values))
+
+
+@pytest.mark.parametrize("missing", ["_raw_stream", "_raw_device"])
+def test_current_stream_without_torchs_raw_calls(missing, monkeypatch):
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(_contract_mod, missing, None)
+    monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+    assert _contract_mod.current_stream() == 77
+
+
+@pytest.mark.gpu
+def test_current_stream_is_torchs():
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    for stream in streams + streams[:1]:
+        with torch.cuda.stream(stream):
+            assert _contract_mod.current_stream() == stream.cuda_stream
+            assert stream.cuda_stream == torch.cuda.current_stream().cuda_stream
