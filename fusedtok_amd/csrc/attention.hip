@@ -790,13 +790,14 @@ void attn_decode_stream(
 // staging (32 rows x 128 B each; chunk c of row w at c ^ ((w >> 1) & 7), so
 // the 16 lanes of a write - two rows - and of a fragment read - 16 rows, one
 // chunk - hit 16 different 16-byte bank groups), K into the score MFMAs' A
-// operand. bf16 takes V through ds_read_b64_tr_b16 straight into the PV
-// product's A (no transposing MFMAs): source lane s of group g addresses V row
-// 4g + s / 4 (+ 16), columns 16 db + 4 (s % 4) .. + 3, and lane (d, g) gets
-// keys 4g + i; the weights go in as three bf16 parts, exactly. fp16 parts
-// cannot hold a float32 weight (their least value is 2^-24), so fp16 takes the
-// PV product of float32 below, lane (r, g) reading V[tok 4g + i][4r .. +3] (8
-// bytes; 16 lanes a whole row) from the staging and widening it.
+// operand, V through ds_read_b64_tr_b16 straight into the PV product's (no
+// transposing MFMAs): source lane s of group g addresses V row 4g + s / 4
+// (+ 16) and four of its columns, and lane (d, g) gets keys 4g + i of the d-th
+// of the 16 columns. The weights go in as three parts of the storage type,
+// with all their 24 bits. fp16 parts hold those of a weight from 2^-16 of the
+// running maximum up; a step with a smaller one takes the PV product of
+// float32 below, lane (r, g) reading V[tok 4g + i][4r .. +3] (8 bytes; 16 lanes
+// a whole row) from the staging and widening it.
 //
 // float32: 16-token steps on v_mfma_f32_16x16x4_f32 (A[r][g], B[g][r],
 // C[4g+i][r]), every product and sum float32. K through the staging (chunk c
@@ -816,9 +817,11 @@ void attn_decode_stream(
 // float32 32 / 8 heads, D = 128, one row of 16384 tokens 109 -> 32 us (4.1
 // TB/s); 16 rows of 100-8000 tokens, paged, 447 -> 117 us (4.6 TB/s); bf16,
 // D = 64, 64 such rows 1050 -> 110 us (4.7 TB/s); 4 rows of 128-1024 tokens,
-// bf16, D = 64, 26.8 -> 12.3 us (graph replays); fp16, D = 64, pays ~10% for
-// its float32 PV (64 rows of 100-8000 tokens 116 us, bf16 104). Error against
-// 64 bits, f32: 2.0e-7 where the general kernel has 2.7e-7 (16384 tokens).
+// bf16, D = 64, 26.8 -> 12.3 us (graph replays). fp16, D = 64, 64 rows of 100-
+// 8000 tokens: 105.4 us with every step's weights in parts (two parts, which
+// lost the small weights, took 102), 115.9 with nearly every step on the
+// float32 PV (one key 20 nats above the rest). Error against 64 bits, f32:
+// 2.0e-7 where the general kernel has 2.7e-7 (16384 tokens).
 // ---------------------------------------------------------------------------
 template <typename T, int D>
 struct WideStep {
@@ -851,8 +854,8 @@ void attn_decode_wide(
     int min_seg, int low_seg, int cus) {
     using W = WideStep<T, D>;
     constexpr bool F32 = W::kF32;
-    constexpr bool PV32 = !std::is_same<T, bf16>::value;  // PV on the float32 MFMA
     constexpr bool PAGED = MODE != kRowsContig;
+    using V8 = typename std::conditional_t<F32, Mfma<bf16>, Mfma<T>>::v8;  // (half storage)
     constexpr int kTok = W::kTok, kRows = W::kRows, kRowLanes = W::kRowLanes;
     constexpr int kElems = 16 / (int)sizeof(T);  // elements per 16-byte chunk
     // the merge rows of the 4 waves alias their staging
@@ -996,7 +999,6 @@ void attn_decode_wide(
                     s[0] = x ? s[0] + sum : sum;
                 }
             } else {
-                using V8 = typename Mfma<T>::v8;
 #pragma unroll
                 for (int h = 0; h < W::kTiles; ++h) {
                     s[h] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1030,46 +1032,118 @@ void attn_decode_wide(
                     psum += s[h][i];
                 }
             l_run = l_run * alpha + psum;
-            if constexpr (PV32) {
+            typedef short v4s __attribute__((ext_vector_type(4)));
+            typedef short v8s __attribute__((ext_vector_type(8)));
+            // half storage: A of the PV product, V[tok 4g + i (i < 4), 16 + 4g
+            // + i - 4][column], the lane giving the addresses of columns c .. +
+            // 3 (c % 4 == 0) of row 4g + r / 4 and its second half
+            auto v_frag = [&](int c) {
+                const int w = 4 * g + (r >> 2);
+                const char* lo_p = stg + W::kStage + at(w, c >> 3) + 2 * (c & 7);
+                const char* hi_p = stg + W::kStage + at(w + 16, c >> 3) + 2 * (c & 7);
+                const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) v4s*)(lo_p));
+                const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) v4s*)(hi_p));
+                return v8s{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            };
+            // the PV product on the float32 MFMA: sum[c][i] is head r's dim
+            // 64 hh + 16g + 4i + c
+            auto pv_f32 = [&](int hh, f32x4 (&sum)[4]) {
+                f32x4 odd[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) sum[c] = odd[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int x = 0; x < 4 * W::kTiles; ++x) {  // token 16h + 4g + i
+                    const int h = x >> 2, i = x & 3;
+                    float vv[4];
+                    if constexpr (F32) {
+                        const f32x4 v4 = __builtin_bit_cast(f32x4, vin[i * (D / 64) + hh]);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) vv[c] = v4[c];
+                    } else {
+                        const float4 v4 = St<T>::ld4(reinterpret_cast<const T*>(
+                            stg + W::kStage + at(16 * h + 4 * g + i, r >> 1) + 8 * (r & 1)));
+                        vv[0] = v4.x, vv[1] = v4.y, vv[2] = v4.z, vv[3] = v4.w;
+                    }
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        f32x4& y = i & 1 ? odd[c] : sum[c];
+                        y = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[c], s[h][i], y, 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < 4; ++c) sum[c] += odd[c];
+            };
+            if constexpr (F32) {
                 // the step's own sum first: one rounding a step in acc
 #pragma unroll
                 for (int hh = 0; hh < D / 64; ++hh) {
-                    f32x4 sum[4], odd[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) sum[c] = odd[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int x = 0; x < 4 * W::kTiles; ++x) {  // token 16h + 4g + i
-                        const int h = x >> 2, i = x & 3;
-                        float vv[4];
-                        if constexpr (F32) {
-                            const f32x4 v4 = __builtin_bit_cast(f32x4, vin[i * (D / 64) + hh]);
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) vv[c] = v4[c];
-                        } else {
-                            const float4 v4 = St<T>::ld4(reinterpret_cast<const T*>(
-                                stg + W::kStage + at(16 * h + 4 * g + i, r >> 1) + 8 * (r & 1)));
-                            vv[0] = v4.x, vv[1] = v4.y, vv[2] = v4.z, vv[3] = v4.w;
-                        }
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            f32x4& y = i & 1 ? odd[c] : sum[c];
-                            y = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[c], s[h][i], y, 0, 0, 0);
-                        }
-                    }
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) sum[c] += odd[c];
+                    f32x4 sum[4];
+                    pv_f32(hh, sum);
 #pragma unroll
                     for (int c = 0; c < 4; ++c)
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
                             acc[4 * hh + c][i] = fmaf(acc[4 * hh + c][i], alpha, sum[c][i]);
                 }
+            } else if constexpr (std::is_same<T, f16>::value) {
+                // acc[x][i]: dim 16g + 4x + i. The weights times 2^15 in three
+                // fp16 parts, truncated: all 24 significant bits of a weight
+                // from 2^-16 up (its last bit is 2^-24 or more there). A step
+                // with a smaller one, or whose result is not finite (an infinite
+                // V times a part that is 0), takes the float32 product.
+                unsigned least = ~0u;  // the bits of the least weight that is not 0, less 1
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    least = min(least, __float_as_uint(s[i >> 2][i & 3]) - 1u);
+                f32x4 sum[4];
+                bool done =
+                    __builtin_amdgcn_ballot_w64(least < __float_as_uint(0x1p-16f) - 1u) == 0;
+                if (done) {
+                    V8 pp[3];
+#pragma unroll
+                    for (int i = 0; i < 8; i += 2) {
+                        float a = s[i >> 2][i & 3] * 0x1p15f, b = s[i >> 2][(i & 3) + 1] * 0x1p15f;
+#pragma unroll
+                        for (int x = 0; x < 3; ++x) {
+                            const auto hi = __builtin_amdgcn_cvt_pkrtz(a, b);
+                            pp[x][i] = (T)hi[0];
+                            pp[x][i + 1] = (T)hi[1];
+                            a -= (float)hi[0];
+                            b -= (float)hi[1];
+                        }
+                    }
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        sum[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        const V8 va = __builtin_bit_cast(V8, v_frag(16 * (r & 3) + 4 * x));
+#pragma unroll
+                        for (int y = 0; y < 3; ++y) sum[x] = Mfma<T>::mma(va, pp[y], sum[x]);
+                    }
+                    // (finite ones are below 2^37: their sum is too)
+                    const f32x4 t = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+                    const float z = (t[0] + t[1]) + (t[2] + t[3]);
+                    done = __builtin_amdgcn_ballot_w64(!(fabsf(z) < INFINITY)) == 0;
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) sum[x] *= 0x1p-15f;
+                }
+                if (!done) {
+                    f32x4 wide[4];
+                    pv_f32(0, wide);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) sum[x][i] = wide[i][x];
+                }
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[x][i] = fmaf(acc[x][i], alpha, sum[x][i]);
             } else {
+                // acc[db][i]: dim 16 db + 4g + i
 #pragma unroll
                 for (int nn = 0; nn < D / 16; ++nn) acc[nn] *= alpha;
-                using V8 = typename Mfma<T>::v8;
-                typedef short v4s __attribute__((ext_vector_type(4)));
-                typedef short v8s __attribute__((ext_vector_type(8)));
                 // the weights in three bf16 parts, truncated: all 24 significant
                 // bits. No part is 0 unless the weight is (exp2f here has no
                 // subnormal results, so its first part is not), so every
@@ -1089,16 +1163,7 @@ void attn_decode_wide(
                 }
 #pragma unroll
                 for (int db = 0; db < D / 16; ++db) {
-                    const int w = 4 * g + (r >> 2);
-                    const int c = 2 * db + ((r & 3) >> 1);
-                    const char* lo_p = stg + W::kStage + at(w, c) + 8 * (r & 1);
-                    const char* hi_p = stg + W::kStage + at(w + 16, c) + 8 * (r & 1);
-                    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) v4s*)(lo_p));
-                    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) v4s*)(hi_p));
-                    const V8 va = __builtin_bit_cast(
-                        V8, v8s{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+                    const V8 va = __builtin_bit_cast(V8, v_frag(16 * db + 4 * (r & 3)));
 #pragma unroll
                     for (int x = 0; x < 3; ++x)
                         acc[db] = Mfma<T>::mma(va, pp[x], acc[db]);
@@ -1142,9 +1207,10 @@ void attn_decode_wide(
         for (int nn = 0; nn < D / 16; ++nn)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                // acc[4h + c][i] of the float32 PV: dim 64h + 16g + 4i + c
-                const int d = PV32 ? 64 * (nn >> 2) + 16 * g + 4 * i + (nn & 3)
-                                  : 16 * nn + 4 * g + i;
+                // the dim of acc[nn][i] (the PV products)
+                const int d = F32 ? 64 * (nn >> 2) + 16 * g + 4 * i + (nn & 3)
+                              : std::is_same<T, f16>::value ? 16 * g + 4 * nn + i
+                                                            : 16 * nn + 4 * g + i;
                 s_acc[wave][r][d] = acc[nn][i];
             }
         __syncthreads();

@@ -692,10 +692,12 @@ def _decode_f64(q, k, v, lens):
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("segs", [0, 1])
-def test_wide_decode_small_weights_count_as_much_as_they_weigh(dt, segs, tuning):
+@pytest.mark.parametrize("gaps", [(17, 20, 25, 32), (10.5, 11, 11.25, 12)])
+def test_wide_decode_small_weights_count_as_much_as_they_weigh(dt, segs, gaps, tuning):
     # four keys (one in each wave's first step) far above the 8188 others,
     # with V = 0 there and V = vbig elsewhere: the output is the sum of the
-    # small weights, 17 to 32 nats below the dominant ones. Scores are exact
+    # small weights, so many nats below the dominant ones (fp16's weights go in
+    # parts down to 2^-16, 11.09 nats). Scores are exact
     # products of one dim (q0 * k0, at most 2^9), so the weights are off by
     # float32's rounding of the exponent (|s| log2(e) 2^-24 < 2^-14 with a
     # margin of two) and the output by the storage rounding: 2^-p for p
@@ -704,8 +706,7 @@ def test_wide_decode_small_weights_count_as_much_as_they_weigh(dt, segs, tuning)
     d, n, hkv, group = 64, 8192, 2, 4
     q = np.zeros((1, hkv * group, d), np.float32)
     k = np.zeros((1, hkv, n, d), np.float32)
-    gaps = np.array([17, 20, 25, 32], np.float32)
-    q[0, :, 0] = np.tile(8 * gaps / 16, hkv)   # s = k0 * gap / 16
+    q[0, :, 0] = np.tile(np.array(gaps, np.float32) / 2, hkv)  # s = k0 * gap / 16
     k[0, :, (0, 32, 64, 96), 0] = 16.0
     vbig = np.array([1.0, 3e4], np.float32)[:, None, None]
     v = np.broadcast_to(vbig, (hkv, n, d)).copy()[None]
