@@ -325,8 +325,8 @@ constexpr int kStreamMinSeg = 512;
 // A call too small to give every CU that many takes shorter segments, one
 // per CU, down to this (bf16, 4 rows of 10-2000 tokens, 8 kv heads: 13.6 us
 // against 22.5 with 512 tokens) - or to half of it where those still leave
-// CUs idle (D = 64, 4 rows of 10-200 tokens, 2.3k flat tokens: bf16 14.2
-// against 18.1 us, fp16 15.9 against 20.7). The line is where 64-token
+// CUs idle (bf16, D = 64, 4 rows of 10-200 tokens, 2.3k flat tokens: 14.2
+// against 18.1 us). The line is where 64-token
 // segments fill the CUs; near it 128 is the better (13.5k flat tokens, bf16,
 // D = 64: 10.9 against 11.6 us).
 constexpr int kStreamLowSeg = 128;

@@ -469,16 +469,18 @@ struct RmsqIo {
     bool store_x = true;  // false: the one-launch form need not store x_out
 };
 
-// Rows (workgroups) of the one-launch form. From 5 rows (rmsq_small takes
-// fewer): in a graph replay the two forms measure the same (5 x 2048 bf16
-// 5.0 us with one launch, 5.3 with two; 16 x 4096 5.7 / 5.6; C4's layer at 64
-// rows 434.6-438.3 against 437.4-438.7: the kernel boundary a replay pays
-// costs about the three dependent device-scope atomic round trips of
-// grid_max), and an eager call saves a launch (10.6 against 13.3 us).
-// Up to 64: the arrivals meet on one counter, one after the other (cols =
-// 4096, bf16 with a residual, graph replays, one launch against two: 64 rows
-// 6.4 / 6.0 us, 128 7.3 / 6.2, 256 9.0 / 7.0, 1000 29.5 / 13.6, 2048 97 / 22;
-// the layer's folded form at 64 rows gains from not storing its input).
+// Rows (workgroups) of the one-launch form, from 5 (rmsq_small takes fewer).
+// It is for eager calls, which save a launch: 10.8 us against 13.5 with two,
+// whatever the rows. A graph replay, whose kernel boundary costs about the
+// three dependent device-scope atomic round trips of grid_max, sees little of
+// it (bf16, one launch / two: 5 x 2048 4.6 / 4.7 us, 5 x 4096 4.7 / 4.8, 8 x
+// 4096 5.0 / 5.0, 16 x 4096 5.2 / 5.0, 64 x 4096 5.8 / 5.1), and pays more
+// with every row, since the arrivals meet on one counter one after the other
+// (with a residual 64 rows 6.4 / 6.0, 128 7.3 / 6.2, 256 9.0 / 7.0, 1000 29.5
+// / 13.6, 2048 97 / 22). The line is at 64 rows: the decode layer's folded
+// form still gains there, also replayed, from not storing its input (C4's
+// layer 434.6-438.3 us against 437.4-438.7), and further up a replay would
+// lose half of what an eager call gains.
 constexpr int kRmsqGridMinRows = 5;
 constexpr int kRmsqGridRows = 64;
 constexpr int kRmsqGridMost = 4096;  // where there is no room for the row statistics
@@ -723,10 +725,11 @@ __global__ __launch_bounds__(kFNT) void swq_quant(
 
 // Both passes in one launch for a step's few elements (4 a thread): the
 // maximum folded with grid_max, the codes from the registers. Every workgroup
-// resident at once, at most kSwqGridWgs of them: from there the arrivals on
-// the one counter cost a graph replay more than the second launch (bf16, one
-// launch against two, us: 4 x 2816, 11 workgroups, 5.1 / 5.5; 6 x 8192, 48,
-// 5.6 / 5.7; 8 x 8192, 64, 5.9 / 5.6); an eager call saves 2.8 us of host time.
+// resident at once, at most kSwqGridWgs of them. An eager call saves 2.5 us of
+// host time at any size (10.6 against 13.1); the line is where a graph replay,
+// which has no such time, stops gaining, so that neither loses (bf16, one
+// launch / two, us: 3 workgroups 4.3 / 4.6, 11 4.7 / 5.0, 32 4.9 / 5.1, 48 5.1
+// / 5.1, 64 5.9 / 5.6: the arrivals on the one counter).
 constexpr int kSwqGridWgs = 48;
 
 template <typename T>
